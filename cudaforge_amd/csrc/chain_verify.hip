@@ -3,12 +3,13 @@
 // One call verifies B sequences of K draft tokens against the target model:
 //   stats   : one streaming pass over the target [B,K+1,V] and draft [B,K,V]
 //             logits -> per-row (max, sum exp) partials (logits input only);
-//   decide  : one wave per sequence gathers p/q at the draft tokens and runs
-//             the acceptance walk (speculative.cpp:66-97 or
-//             speculative.py:155-185), leaving at most one draw per row;
-//   sample  : one work-group per sequence performs that draw with the exact
-//             sequential-fp32 inverse CDF of speculative.cpp:11-48
-//             (seqsum.hpp), then writes the outputs.
+//   decide  : p/q gathered at the draft tokens and the acceptance walk
+//             (speculative.cpp:66-97, inside the first draw kernel, or
+//             speculative.py:155-185, py_decide_kernel), leaving at most one
+//             draw per row;
+//   draw    : the exact sequential-fp32 inverse CDF of speculative.cpp:11-48
+//             (seqsum.hpp) over many work-groups, which ends by writing the
+//             outputs.
 // Greedy mode (speculative.cpp:105-150) replaces sample by a first-argmax pass.
 //
 // Probabilities computed from logits (the fused path) are
@@ -56,11 +57,12 @@ struct MwJob {  // what sequence b still has to draw
   float dM, dInvS;  // and of the draft row of a residual draw
   int extra;        // python mode: a bonus draw follows the resample
   float u2;         // and its threshold
-  int pad;
+  float vstar;      // a bonus draw's smallest kept probability
 };
-struct MwRes {  // per sequence: residual sum, fallback flag, drawn index(es)
+struct MwRes {  // per sequence: residual sum, fallback flag, drawn index
   float S;
-  int fallback, idx, idx2;
+  int fallback, idx;
+  int nmin;  // python mode, entry 0: the batch's accept count
 };
 struct MwRec {  // a tile's function of the entry parity, its region guess, pad = 1: replay
   uint32_t e, o;
@@ -80,6 +82,15 @@ struct MwChunk {
 struct MwBad {  // a tile the walk will probably replay serially, with its values
   int tile, pad[3];
   float x[kMwTile];
+};
+// What select_kernel found of a row's smallest kept probability v: it lies in
+// histogram bin `bin` (or is known: state kSelKnown, its bits in `bin`),
+// F and C are the sum and the count of the probabilities in higher bins, and
+// the rules still open (bit 0 top-p, bit 1 top-k) are in `rules`.
+struct SelRow {
+  double F;
+  uint32_t C;
+  uint16_t bin, rules;
 };
 
 struct Args {
@@ -105,10 +116,10 @@ struct Args {
   int P;         // cpp rules, logits: positions whose rows the first stats pass reads
   float2 *part;  // [R, S] (max logit, sum exp) per (row, slice)
   float2 *apart; // [R, S] (max prob, index as bits) per (row, slice)
-  int4 *dec;     // [B] {n_b, kind, row, eos_accepted}
-  float *ufin;   // [B]
+  // python mode
+  int *nmin;     // the batch's accept count, min_b n_b (speculative.py:166)
+  float2 *rstat; // [R] (max, 1/S) of every row, from py_decide_kernel
   // exact multi-work-group sampler (see "mw" below)
-  int vec;                // rows are 16-byte aligned with V % 4 == 0
   int NC;                 // chunks per row
   MwJob *jobs;            // [B]
   MwRes *res;             // [B]
@@ -123,6 +134,10 @@ struct Args {
   float *s0;              // [B] sum pass: the exact running value after chunk 0
   int mw_reset;           // the first statistics pass zeroes flags and badcnt
   float *rawtok;          // [R] head pass: a row's raw logit at its position's draft token
+  // smallest kept probability of the bonus rows (see "kept probabilities")
+  int HG;                 // histogram slices per row (1: a short row, 0: nothing is filtered)
+  SelRow *sel;            // [groups]
+  int *lcnt;              // [groups] keys listed (more than the capacity: not all of them)
   int32_t *out_accept_len, *out_tokens, *out_num_emitted, *out_final, *out_eos;
 };
 
@@ -177,6 +192,39 @@ __device__ float2 row_stat(const Args &a, int r) {
   return make_float2(M, 1.0f / S);
 }
 
+// The same by one wave (every lane gets it): the partials load in one round,
+// and their terms are added in slice order.
+__device__ float2 wave_row_stat(const Args &a, int r) {
+  constexpr int kQ = 4;  // stats_slices: at most 256 slices
+  const int lane = threadIdx.x & 63;
+  const float2 *p = a.part + (long long)r * a.S;
+  float2 q[kQ];
+#pragma unroll
+  for (int k = 0; k < kQ; ++k)
+    q[k] = 64 * k + lane < a.S ? p[64 * k + lane] : make_float2(-INFINITY, 0.0f);
+  float M = fmaxf(fmaxf(q[0].x, q[1].x), fmaxf(q[2].x, q[3].x));
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) M = fmaxf(M, __shfl_xor(M, d, 64));
+  float S = 0.0f;
+#pragma unroll
+  for (int k = 0; k < kQ; ++k) {
+    const float t = (q[k].x == M) ? q[k].y : q[k].y * __builtin_amdgcn_exp2f((q[k].x - M) * a.c);
+    const int n = min(64, a.S - 64 * k);
+    for (int w = 0; w < n; ++w) S += u2f((uint32_t)__builtin_amdgcn_readlane((int)f2u(t), w));
+  }
+  return make_float2(M, 1.0f / S);
+}
+
+// Row j of job b without its statistics.
+__device__ __forceinline__ Dist make_raw_dist(const Args &a, int b, int j) {
+  Dist d;
+  d.p = row_ptr(a, b, j);
+  d.c = a.c;
+  d.logits = a.logits;
+  d.M = 0.0f;
+  d.invS = 1.0f;
+  return d;
+}
 __device__ Dist make_dist_u(const Args &a, int ub, int j) {
   Dist d;
   d.p = row_ptr_u(a, ub, j);
@@ -233,11 +281,12 @@ __device__ __forceinline__ float4 ld_stream4(const float4 *p) {
   return make_float4(q[0], q[1], q[2], q[3]);
 }
 
-// Row sets of a stats pass.  Under the cpp rules with logits input only the
-// rows of positions up to a sequence's first rejection are ever read, so
-// the first pass takes positions 0 .. P-1 of every sequence ("head"), and
+// Row sets of a stats pass.  With logits input only the rows of positions up
+// to a sequence's first rejection (python mode: the batch's) are ever read,
+// so the first pass takes positions 0 .. P-1 of every sequence ("head"), and
 // the second the remaining rows (positions P .. K-1 and the target's row K,
-// "tail") of the sequences that accepted all P head positions.
+// "tail") of the sequences that accepted all P head positions (python mode:
+// of all of them or of none).
 enum RowSet : int { kRowsAll = 0, kRowsHead = 1, kRowsTail = 2 };
 
 // Row id (ub * rpb + j) of entry y of a row set; -1 past its end.
@@ -253,9 +302,17 @@ __device__ __forceinline__ int set_row(const Args &a, int set, int y) {
   return ub < groups ? ub * a.rpb + (q <= K - P ? P + q : K + 1 + P + (q - (K - P + 1))) : -1;
 }
 
-// Whether row group ub accepted head position i under the cpp rules
-// (speculative.cpp:66-80: position i takes the i-th uniform when all before
-// it were accepted, and an accepted EOS ends the walk), from the head pass's
+// Whether a position with draft token traw is accepted and verification goes
+// on past it: the cpp rules (speculative.cpp:66-80: position i takes the i-th
+// uniform when all before it were accepted, and an accepted EOS ends the
+// walk) or the python rule (speculative.py:161-164).
+__device__ __forceinline__ bool pos_accepts(const Args &a, int traw, float u, float pt, float qd) {
+  const bool valid = traw >= 0 && traw < a.V;
+  if (a.mode == CFA_MODE_PYTHON) return u < ratio_py(valid ? pt : 0.0f, valid ? qd : 0.0f);
+  return valid && u <= ratio_cpp(pt, qd) && traw != a.eos;
+}
+
+// The same for head position i of row group ub, from the head pass's
 // statistics and the raw logit at the draft token it recorded.
 __device__ __forceinline__ bool head_accepts(const Args &a, int ub, int i) {
   const int rt = ub * a.rpb + i, rd = ub * a.rpb + a.K + 1 + i;
@@ -264,8 +321,7 @@ __device__ __forceinline__ bool head_accepts(const Args &a, int ub, int i) {
   const float2 st = row_stat(a, rt), sd = row_stat(a, rd);
   const float pt = __builtin_amdgcn_exp2f((a.rawtok[rt] - st.x) * a.c) * st.y;
   const float qd = __builtin_amdgcn_exp2f((a.rawtok[rd] - sd.x) * a.c) * sd.y;
-  const bool valid = traw >= 0 && traw < a.V;
-  return valid && u <= ratio_cpp(pt, qd) && traw != a.eos;
+  return pos_accepts(a, traw, u, pt, qd);
 }
 
 // Whether row group ub accepted every head position (head_accepts for each,
@@ -301,8 +357,7 @@ __device__ bool head_all_accept(const Args &a, int ub) {
       const float2 st = row_parts_stat(a, qt[i]), sd = row_parts_stat(a, qd[i]);
       const float pt = __builtin_amdgcn_exp2f((rt[i] - st.x) * a.c) * st.y;
       const float q = __builtin_amdgcn_exp2f((rd[i] - sd.x) * a.c) * sd.y;
-      const bool valid = tk[i] >= 0 && tk[i] < a.V;
-      ok &= valid && u[i] <= ratio_cpp(pt, q) && tk[i] != a.eos;
+      ok &= pos_accepts(a, tk[i], u[i], pt, q);
     }
   }
   return ok;
@@ -358,14 +413,21 @@ __device__ __forceinline__ float2 slice_partial(const Args &a, int r, int slice)
       }
     }
   } else {
-    for (long long i = s0 + threadIdx.x; i < s1; i += NT) {
-      const float v = __builtin_nontemporal_load(row + i);
-      if (v > m) {
-        s *= __builtin_amdgcn_exp2f((m - v) * c);
-        m = v;
+    // (rows of any length and alignment: single elements, 4 U loads in flight)
+    for (long long i0 = s0 + threadIdx.x; i0 < s1; i0 += 4 * U * NT) {
+      float v[4 * U];
+#pragma unroll
+      for (int u = 0; u < 4 * U; ++u) v[u] = __builtin_nontemporal_load(row + min(i0 + u * NT, s1 - 1));
+#pragma unroll
+      for (int u = 0; u < 4 * U; ++u) {
+        if (i0 + u * NT >= s1) v[u] = -INFINITY;  // folds nothing, as above
+        if (v[u] > m) {
+          s *= __builtin_amdgcn_exp2f((m - v[u]) * c);
+          m = v[u];
+        }
+        const float ms = (m == -INFINITY) ? 0.0f : m;
+        s += __builtin_amdgcn_exp2f((v[u] - ms) * c);
       }
-      const float ms = (m == -INFINITY) ? 0.0f : m;
-      s += __builtin_amdgcn_exp2f((v - ms) * c);
     }
   }
   return block_ms<NT>(m, s, c);
@@ -409,15 +471,14 @@ __global__ __launch_bounds__(NT) void stats_kernel(Args a, int set) {
 // Row groups the balanced tail pass can list in LDS.
 constexpr int kTailMaxGroups = 4096;
 
-// The tail pass, balanced over the device (16-byte loads; row groups <=
-// kTailMaxGroups).  A grid of one work-group per (tail row, slice) leaves
+// The tail pass, balanced over the device (row groups <= kTailMaxGroups).  A grid of one work-group per (tail row, slice) leaves
 // most work-groups with nothing to do (their sequence rejected a head
 // position), and the CUs that happen to hold several busy ones pace the
 // pass.  Here every work-group lists the groups that need their tail rows
 // (one thread per group) and takes every gridDim.x-th (group, tail row,
 // slice) item of that list, so every CU streams about the same bytes.  Each
 // item's partial is the one stats_kernel computes for that (row, slice).
-template <int NT>
+template <int NT, int W>
 __global__ __launch_bounds__(NT) void stats_tail_kernel(Args a) {
   static_assert(NT == kStatsNT, "every statistics pass folds a slice the same way");
   __shared__ int list[kTailMaxGroups];
@@ -443,13 +504,16 @@ __global__ __launch_bounds__(NT) void stats_tail_kernel(Args a) {
     __syncthreads();
   }
   const int K = a.K, P = a.P, per = 2 * (K - P) + 1;
+  // python mode's lock step: a position past the head is reached by every
+  // group or by none
+  if (a.mode == CFA_MODE_PYTHON && base < groups) return;
   const long long total = (long long)base * per * a.S;
   for (long long k = blockIdx.x; k < total; k += gridDim.x) {
     const int ub = list[k / ((long long)per * a.S)];
     const int rem = (int)(k % ((long long)per * a.S));
     const int q = rem / a.S, slice = rem % a.S;
     const int r = ub * a.rpb + (q <= K - P ? P + q : K + 1 + P + (q - (K - P + 1)));
-    const float2 out = slice_partial<NT, 4, 4>(a, r, slice);
+    const float2 out = slice_partial<NT, W, 4>(a, r, slice);
     if (threadIdx.x == 0) a.part[(long long)r * a.S + slice] = out;
   }
 }
@@ -506,54 +570,110 @@ __device__ int row_argmax(const Args &a, int r) {
 }
 
 // ---------------------------------------------------------------------------
-// decide: one wave per sequence.
+// jobs: the draw each sequence still needs.
+// ---------------------------------------------------------------------------
+
+// Python-mode draws take the first index whose sequential prefix sum
+// EXCEEDS u (so u = 0 never selects a zero-weight entry, as torch.multinomial
+// never does); the inverse-CDF walks test `r <= prefix`, and for floats
+// u < x <=> succ(u) <= x.  The floor FLT_MIN keeps r out of the denormals.
+__device__ __forceinline__ float py_threshold(float u) {
+  // for finite u >= 0 the next float up is the next bit pattern
+  const float s = (u >= 0.0f && u < INFINITY) ? __uint_as_float(__float_as_uint(u) + 1u) : u;
+  return fmaxf(s, 1.17549435e-38f);
+}
+
+// A sequence's job: its draw (n, kind, row, eos_acc, threshold u; a
+// python-mode bonus after the resample when extra) and the statistics of the
+// draw's rows (st: those of the sequence's rows).
+__device__ __forceinline__ MwJob make_job(const Args &a, int n, int kind, int row, int eos_acc, float u,
+                                          int extra, float u2, const float2 *st) {
+  MwJob j;
+  j.n = n;
+  j.kind = kind;
+  j.row = row;
+  j.eos_acc = eos_acc;
+  j.u = u;
+  j.extra = extra;
+  j.u2 = u2;
+  j.vstar = 0.0f;
+  j.tM = j.dM = 0.0f;
+  j.tInvS = j.dInvS = 1.0f;
+  if (a.logits && kind != kNone) {
+    j.tM = st[row].x;
+    j.tInvS = st[row].y;
+    if (kind == kResid) {
+      j.dM = st[a.K + 1 + row].x;
+      j.dInvS = st[a.K + 1 + row].y;
+    }
+  }
+  return j;
+}
+
+// Python mode: the job of b, after py_decide_kernel.  A rejection at the last
+// position (n = K - 1) brings the reference's num_accepted to K, so its
+// `num_accepted == self.k` branch (speculative.py:188-195) appends a bonus
+// draw after the resample.
+__device__ __forceinline__ MwJob py_job(const Args &a, int b) {
+  const int K = a.K, n = *a.nmin;
+  const float *u = a.U + (long long)b * a.ustride + K;
+  const int extra = (K > 0 && n == K - 1) ? 1 : 0;
+  return make_job(a, n, n < K ? kResid : kPyBonus, n, 0, py_threshold(u[0]), extra,
+                  extra ? py_threshold(u[1]) : 0.0f, a.rstat + (long long)(b / a.draws) * a.rpb);
+}
+
+// ---------------------------------------------------------------------------
+// decide: the acceptance rules.
 // ---------------------------------------------------------------------------
 
 constexpr int kMaxK = 64;
 
-struct DecideLds;
-__device__ MwJob make_job(const Args &a, int b, int n, int kind, int row, int eos_acc, float u,
-                         int extra = 0, float u2 = 0.0f, const DecideLds *L = nullptr);
-__device__ void write_job(const Args &a, int b, const MwJob &j);
-
 // The decision's inputs, gathered by a work-group of nt threads: the draft
 // tokens and p(tok), q(tok) at every position with the statistics of every
-// row of the sequence (or, greedy, the first argmax of every target row),
-// and the sequence's uniforms.  One thread per row, so a row's partials and
-// its value at the token are two rounds of loads for the whole gather.
+// row of the sequence, and the sequence's uniforms.  With at most kFastS
+// slices a row, one thread per row (its partials and its value at the token
+// are two rounds of loads for the whole gather); with more, one wave per row
+// (a thread's loop over 31 partials took 8.8 us of a 92 us call at B = 1,
+// V = 32000).
 struct DecideLds {
   float pt[kMaxK], qd[kMaxK];
-  int tk[kMaxK], am[kMaxK + 1], ok[kMaxK];
+  int tk[kMaxK], ok[kMaxK];
   float2 st[2 * kMaxK + 1];  // (max, 1/S) of rows 0 .. 2K (logits input)
   float u[kMaxK + 2];
 };
 
 __device__ void decide_gather(const Args &a, int b, int tid, int nt, DecideLds &L) {
   const int K = a.K;
-  if (a.mode == CFA_MODE_GREEDY) {
-    for (int i = tid; i < K; i += nt) L.tk[i] = a.tokens[(long long)b * K + i];
-    for (int i = tid; i <= K; i += nt) L.am[i] = row_argmax(a, (b / a.draws) * a.rpb + i);
-    return;
-  }
   // rows 0 .. K-1 target at a draft position, K the target's last row,
   // K+1 .. 2K draft
-  for (int r = tid; r < 2 * K + 1; r += nt) {
+  auto put = [&](int r, int i, int traw, bool valid, float raw, const Dist &d) {
+    L.st[r] = make_float2(d.M, d.invS);
+    if (r == K) return;
+    const float v = valid ? d.eval(raw) : 0.0f;
+    if (r < K) {
+      L.pt[i] = v;
+      L.tk[i] = traw;
+      L.ok[i] = valid ? 1 : 0;
+    } else {
+      L.qd[i] = v;
+    }
+  };
+  const bool by_wave = a.logits && a.S > kFastS;
+  const int step = by_wave ? nt / 64 : nt;
+  for (int r = by_wave ? tid / 64 : tid; r < 2 * K + 1; r += step) {
     const int i = r <= K ? r : r - K - 1;
     const int traw = (r != K) ? a.tokens[(long long)b * K + i] : 0;
-    const Dist d = make_dist(a, b, r);
-    L.st[r] = make_float2(d.M, d.invS);
-    if (r != K) {
-      const int t = min(max(traw, 0), a.V - 1);  // never read outside the row
-      const bool valid = traw == t;                // an id outside [0, V) is never accepted
-      const float v = valid ? d(t) : 0.0f;
-      if (r < K) {
-        L.pt[i] = v;
-        L.tk[i] = traw;
-        L.ok[i] = valid ? 1 : 0;
-      } else {
-        L.qd[i] = v;
-      }
+    const int t = min(max(traw, 0), a.V - 1);  // never read outside the row
+    const bool valid = traw == t;                // an id outside [0, V) is never accepted
+    Dist d = make_raw_dist(a, b, r);
+    const float raw = d.load(t);
+    if (a.logits) {
+      const int row = (b / a.draws) * a.rpb + r;
+      const float2 st = by_wave ? wave_row_stat(a, row) : row_stat(a, row);
+      d.M = st.x;
+      d.invS = st.y;
     }
+    if (!by_wave || (tid & 63) == 0) put(r, i, traw, valid, raw, d);
   }
   const int nu = min(a.ustride, kMaxK + 2);
   for (int i = tid; i < nu; i += nt) L.u[i] = a.U[(long long)b * a.ustride + i];
@@ -586,53 +706,54 @@ __device__ MwJob decide_cpp(const Args &a, int b, const DecideLds &L) {
     row = K;
     uf = L.u[draws++];
   }
-  return make_job(a, b, n, kind, row, eos_acc, uf, 0, 0.0f, &L);
+  return make_job(a, n, kind, row, eos_acc, uf, 0, 0.0f, L.st);
 }
 
-// One work-group per sequence.  cpp mode runs this only where the exact
-// draw is not needed (the mw sums kernel decides otherwise); python mode
-// records n_b for plan_kernel; greedy writes the final outputs.
+// Python mode, one work-group per row group: its accept count n_b into the
+// batch's minimum (the lock-step rule of speculative.py:166; the first kernel
+// of the call sets it to K) and its rows' statistics, from which every later
+// kernel forms its jobs (py_job).  One wave per row.
+__global__ __launch_bounds__(1024) void py_decide_kernel(Args a) {
+  const int ub = blockIdx.x, K = a.K;
+  __shared__ DecideLds L;
+  decide_gather(a, ub * a.draws, threadIdx.x, blockDim.x, L);
+  __syncthreads();
+  if (a.logits)
+    for (int r = threadIdx.x; r < a.rpb; r += blockDim.x) a.rstat[(long long)ub * a.rpb + r] = L.st[r];
+  if (threadIdx.x != 0 || K == 0) return;
+  int n = K;
+  for (int i = K - 1; i >= 0; --i)
+    if (!(L.u[i] < ratio_py(L.pt[i], L.qd[i]))) n = i;
+  if (n < K) atomicMin(a.nmin, n);
+}
+
+// Greedy: one wave per sequence writes its outputs.
 __global__ __launch_bounds__(64) void decide_kernel(Args a) {
   const int b = blockIdx.x, lane = threadIdx.x;
-  __shared__ DecideLds L;
+  __shared__ int tk[kMaxK], am[kMaxK + 1];
   const int K = a.K;
-  decide_gather(a, b, lane, 64, L);
+  for (int i = lane; i < K; i += 64) tk[i] = a.tokens[(long long)b * K + i];
+  for (int i = lane; i <= K; i += 64) am[i] = row_argmax(a, b * a.rpb + i);
   __syncthreads();
   if (lane != 0) return;
-  if (a.mode == CFA_MODE_CPP) {
-    write_job(a, b, decide_cpp(a, b, L));
-    return;
-  }
   int n = 0, eos_acc = 0;
-  if (a.mode == CFA_MODE_PYTHON) {
-    n = K;
-    for (int i = 0; i < K; ++i)
-      if (!(L.u[i] < ratio_py(L.pt[i], L.qd[i]))) {
-        n = i;
-        break;
-      }
-    a.dec[b] = make_int4(n, kNone, -1, 0);
-    a.ufin[b] = L.u[K];
-    return;
-  }
-  // greedy: outputs are final here
   int fin = -1;
   for (int i = 0; i < K; ++i) {
-    if (L.tk[i] == L.am[i]) {
+    if (tk[i] == am[i]) {
       ++n;
-      if (L.tk[i] == a.eos) {
+      if (tk[i] == a.eos) {
         eos_acc = 1;
         fin = a.eos;
         break;
       }
     } else {
-      fin = L.am[i];
+      fin = am[i];
       break;
     }
   }
-  if (!eos_acc && n == K) fin = L.am[K];
+  if (!eos_acc && n == K) fin = am[K];
   int32_t *ot = a.out_tokens + (long long)b * (K + 1);
-  for (int j = 0; j <= K; ++j) ot[j] = (j < n) ? L.tk[j] : -1;
+  for (int j = 0; j <= K; ++j) ot[j] = (j < n) ? tk[j] : -1;
   if (!eos_acc) ot[n] = fin;
   a.out_accept_len[b] = n;
   a.out_final[b] = fin;
@@ -644,21 +765,6 @@ __global__ __launch_bounds__(64) void decide_kernel(Args a) {
 // sample: one work-group per sequence, exact sequential inverse CDF.
 // ---------------------------------------------------------------------------
 
-struct XResid {  // max(0, t_i - d_i)            (speculative.cpp:33)
-  Dist t, d;
-  using Raw = float2;
-  __device__ __forceinline__ Raw load(long long i) const { return make_float2(t.load(i), d.load(i)); }
-  __device__ __forceinline__ float eval(Raw v) const { return relu_ref(t.eval(v.x) - d.eval(v.y)); }
-};
-struct XResidNorm {  // max(0, t_i - d_i) / sum    (speculative.cpp:44)
-  Dist t, d;
-  float S;
-  using Raw = float2;
-  __device__ __forceinline__ Raw load(long long i) const { return make_float2(t.load(i), d.load(i)); }
-  __device__ __forceinline__ float eval(Raw v) const {
-    return relu_ref(t.eval(v.x) - d.eval(v.y)) / S;
-  }
-};
 struct XKeep {  // top-p kept probabilities (speculative.py:67-83)
   Dist t;
   float vstar;
@@ -680,133 +786,363 @@ struct XKeepNorm {
   }
 };
 
-template <int NT>
-__device__ double block_sum_f64(double v, double *red) {
+// ---------------------------------------------------------------------------
+// Kept probabilities of the python-mode bonus and the filtered sampler: those
+// >= v, the larger of
+//   top-p  the least v with sum_{p_i > v} p_i <= top_p (fp64 sums;
+//          speculative.py:67-81), and
+//   top-k  the least v with #{p_i > v} < top_k (ties kept).
+// Probabilities order as their fp32 bits ("keys"), so both are radix
+// selections:
+//   hist_kernel    per slice of the row, the count and fp64 sum of the
+//                  probabilities of every 2^20-key bin (8 bins a binade);
+//   select_kernel  sums the slices' bins, walks them from the top to the bin
+//                  that holds v, and lists that bin's keys;
+//   sel_finish     two more 10-bit levels over the listed keys, by every
+//                  work-group that needs v.
+// A row shorter than kSelMinNC chunks has no room for the bins in the
+// workspace (they share the first exact pass's tile records, the keys the
+// second's, both written later): select_short_kernel, one work-group per row,
+// keeps its bins in LDS instead.
+// Before, one work-group per row bisected v over the key bits, up to 62
+// passes over the row: 1284 us for 32 rows of V = 128256 (top-k 50 and
+// top-p 0.9), bound by one CU's exponentials per row.
+// ---------------------------------------------------------------------------
+
+constexpr int kSelBins = 1024;
+constexpr int kSelShift = 20;
+constexpr int kSelMaxList = 8192;
+constexpr int kSelNT = 1024;
+constexpr int kSelBytes = kSelBins * 12;  // a slice's bins in the workspace
+constexpr int kSelMinNC = 2 * kSelBytes / (kMwChunkTiles * (int)sizeof(MwRec));  // two slices' room
+constexpr int kSelMaxHG = 16;
+enum SelRules : int { kRuleP = 1, kRuleK = 2, kSelKnown = 4 };
+
+struct SelLds {
+  double sum[kSelBins];
+  uint32_t cnt[kSelBins];
+  double wF[16];
+  uint32_t wC[16];
+  int wbp[16], wbk[16], wlow[16];
+  double F;
+  uint32_t C;
+};
+
+__device__ __forceinline__ int sel_rules(const Args &a) {
+  return (a.top_p < 1.0f ? kRuleP : 0) | (a.top_k > 0 && a.top_k < a.V ? kRuleK : 0);
+}
+
+// Probabilities at or below this cannot be v.  All V of them together sum to
+// at most 0.9 (1 - top_p), and the row's sum is 1 to within 1e-5 (softmax of
+// the same fp32 values), so what lies above sums to more than top_p; the
+// bound is only used where 0.1 (1 - top_p) is well above that 1e-5.
+__device__ __forceinline__ float sel_floor(const Args &a) {
+  return (a.logits && a.top_p <= 0.999f) ? 0.9f * (1.0f - a.top_p) / (float)a.V : 0.0f;
+}
+
+__device__ __forceinline__ int sel_bin(uint32_t key) {
+  return (int)min(key >> kSelShift, (uint32_t)(kSelBins - 1));
+}
+
+// Every key above `lo` (never NaN, zero or negative) of elements [e0, e1) of
+// row t to fn(key), by a work-group of NT threads.  (Small unrolls: the
+// selection kernels run their code about once per wave, so instruction
+// fetches count; 32 elements a batch instead of 4 took select_kernel from 22
+// to 30 us.)
+template <int NT, class Fn>
+__device__ __forceinline__ void sel_scan_row(const Dist &t, long long e0, long long e1, float lo,
+                                             const Fn &fn) {
+  constexpr int U = 8;
+#pragma unroll 1
+  for (long long i0 = e0 + threadIdx.x; i0 < e1; i0 += U * NT) {
+    float v[U];
 #pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d, 64);
+    for (int u = 0; u < U; ++u) v[u] = t.load(min(i0 + u * NT, e1 - 1));
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const float p = t.eval(v[u]);
+      if (i0 + u * NT < e1 && p > lo) fn(f2u(p));
+    }
+  }
+}
+
+template <int NT>
+__device__ __forceinline__ void sel_zero(SelLds &L) {
+  for (int i = threadIdx.x; i < kSelBins; i += NT) {
+    L.sum[i] = 0.0;
+    L.cnt[i] = 0;
+  }
+  __syncthreads();
+}
+
+__device__ __forceinline__ void sel_add(SelLds &L, int bin, uint32_t key, bool sums) {
+  atomicAdd(&L.cnt[bin], 1u);
+  if (sums) unsafeAtomicAdd(&L.sum[bin], (double)u2f(key));
+}
+
+// The bin of L (complete, synchronised) that holds v, given the sum F and
+// count C of everything above the bins and the open rules; updates F, C and
+// rules to what holds inside that bin.  -1: no bin does (every probability
+// is kept); with `inside` (v is known to lie in these bins) the lowest
+// non-empty bin instead.  All NT threads; L is free again on return.
+template <int NT>
+__device__ int sel_find(SelLds &L, const Args &a, double &F, uint32_t &C, int &rules, bool inside) {
+  constexpr int BPT = kSelBins / NT;  // thread t owns BPT bins, t = 0 the highest
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int top = kSelBins - 1 - (int)threadIdx.x * BPT;
+  double f = 0.0;
+  uint32_t c = 0;
+#pragma unroll
+  for (int k = 0; k < BPT; ++k) {
+    f += L.sum[top - k];
+    c += L.cnt[top - k];
+  }
+  double fi = f;
+  uint32_t ci = c;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const double fo = __shfl_up(fi, d, 64);
+    const uint32_t co = __shfl_up(ci, d, 64);
+    if (lane >= d) {
+      fi += fo;
+      ci += co;
+    }
+  }
+  if (lane == 63) {
+    L.wF[wave] = fi;
+    L.wC[wave] = ci;
+  }
   __syncthreads();
-  if (lane == 0) red[wave] = v;
+  constexpr int NW = NT / 64;
+  double fx = F + (fi - f);
+  uint32_t cx = C + (ci - c);
+#pragma unroll
+  for (int w = 0; w < NW; ++w) {
+    fx += w < wave ? L.wF[w] : 0.0;
+    cx += w < wave ? L.wC[w] : 0u;
+  }
+  // each rule's first (highest) bin past it, and the lowest non-empty bin:
+  // per thread, then per wave by ballot (an LDS maximum over every thread
+  // past the crossing cost 8 us), then over the waves
+  double fr = fx;
+  uint32_t cr = cx;
+  int bp = -1, bk = -1, low = -1;
+#pragma unroll
+  for (int k = 0; k < BPT; ++k) {
+    fr += L.sum[top - k];
+    cr += L.cnt[top - k];
+    if ((rules & kRuleP) && bp < 0 && fr > (double)a.top_p) bp = top - k;
+    if ((rules & kRuleK) && bk < 0 && cr >= (uint32_t)a.top_k) bk = top - k;
+    if (L.cnt[top - k]) low = top - k;
+  }
+  const unsigned long long mp = __ballot(bp >= 0), mk = __ballot(bk >= 0), ml = __ballot(low >= 0);
+  const int wbp = mp ? __builtin_amdgcn_readlane(bp, (int)__builtin_ctzll(mp)) : -1;
+  const int wbk = mk ? __builtin_amdgcn_readlane(bk, (int)__builtin_ctzll(mk)) : -1;
+  const int wlow = ml ? __builtin_amdgcn_readlane(low, 63 - (int)__builtin_clzll(ml)) : -1;
+  if (lane == 0) {
+    L.wbp[wave] = wbp;
+    L.wbk[wave] = wbk;
+    L.wlow[wave] = wlow;
+  }
   __syncthreads();
-  double t = 0.0;
-  for (int w = 0; w < NT / 64; ++w) t += red[w];
+  bp = bk = low = -1;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) {
+    bp = max(bp, L.wbp[w]);
+    bk = max(bk, L.wbk[w]);
+    low = L.wlow[w] >= 0 ? L.wlow[w] : low;
+  }
+  int bin = max(bp, bk);
+  const int r2 = ((rules & kRuleP) && bp == bin ? kRuleP : 0) | ((rules & kRuleK) && bk == bin ? kRuleK : 0);
+  if (bin < 0 && inside) bin = max(low, 0);  // the crossing was lost to fp64 rounding
+  if (bin >= 0 && bin <= top && bin > top - BPT) {
+    for (int k = 0; top - k > bin; ++k) {
+      fx += L.sum[top - k];
+      cx += L.cnt[top - k];
+    }
+    L.F = fx;
+    L.C = cx;
+  }
+  __syncthreads();
+  if (bin >= 0) {
+    F = L.F;
+    C = L.C;
+    if (r2) rules = r2;
+  }
+  __syncthreads();
+  return bin;
+}
+
+// v from the bin that holds it: a radix selection of the bin's keys, 10 bits
+// a level.  The keys are list[0 .. n - 1], or with list == nullptr those of
+// row t (n elements).  bin < 0: the bins are still to be made, too, at the
+// first level (from the row).
+template <int NT>
+__device__ float sel_levels(SelLds &L, const Args &a, double F, uint32_t C, int rules, int bin,
+                            const uint32_t *list, const Dist &t, int n) {
+  const float lo = sel_floor(a);
+  const uint32_t *src = list ? list : reinterpret_cast<const uint32_t *>(t.p);
+  uint32_t pre = 0;
+  // (the last bin is open above: its keys differ in 30 bits)
+  int shift = bin < 0 ? kSelShift : bin == kSelBins - 1 ? 20 : 10;
+#pragma unroll 1
+  while (shift >= 0) {
+    sel_zero<NT>(L);
+    const bool sums = (rules & kRuleP) != 0;
+    const uint32_t base = (uint32_t)max(bin, 0) << kSelShift;
+    constexpr int U = 8;
+#pragma unroll 1
+    for (int i0 = threadIdx.x; i0 < n; i0 += U * NT) {
+      uint32_t k[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) k[u] = src[min(i0 + u * NT, n - 1)];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (!list) {
+          const float p = t.eval(u2f(k[u]));
+          k[u] = (p > lo && (bin < 0 || sel_bin(f2u(p)) == bin)) ? f2u(p) : 0u;
+        }
+        const uint32_t rel = (k[u] - base) >> shift;
+        if (i0 + u * NT < n && k[u] != 0u && (bin < 0 || rel >> 10 == pre))
+          sel_add(L, (int)(bin < 0 ? min(rel, (uint32_t)(kSelBins - 1)) : rel & (kSelBins - 1)), k[u], sums);
+      }
+    }
+    __syncthreads();
+    const int q = sel_find<NT>(L, a, F, C, rules, bin >= 0);
+    if (bin < 0) {
+      if (q < 0) return u2f(1u);  // no rule cuts anything: every positive probability is kept
+      bin = q;
+      shift = bin == kSelBins - 1 ? 20 : 10;
+      continue;
+    }
+    pre = (pre << 10) | (uint32_t)q;
+    shift -= 10;
+  }
+  return u2f(((uint32_t)bin << kSelShift) + pre);
+}
+
+// The capacity of a row's key list, and the list.
+__device__ __forceinline__ int sel_cap(const Args &a) {
+  return min(kSelMaxList, a.NC * kMwChunkTiles * (int)(sizeof(MwRec) / sizeof(uint32_t)));
+}
+__device__ __forceinline__ uint32_t *sel_list(const Args &a, int ub) {
+  return reinterpret_cast<uint32_t *>(a.trec + ((long long)a.B + (long long)ub * a.draws) * a.NC * kMwChunkTiles);
+}
+__device__ __forceinline__ unsigned char *sel_hist(const Args &a, int ub) {
+  return reinterpret_cast<unsigned char *>(a.trec + (long long)ub * a.draws * a.NC * kMwChunkTiles);
+}
+
+// The bonus row of group ub with its statistics.  `first`: with K = 0 (the
+// sampler, which has nothing to decide) the first selection kernel forms
+// them in py_decide_kernel's place, every wave for itself, and the
+// work-group with store set keeps them for the kernels after it.
+__device__ Dist sel_dist(const Args &a, int ub, bool first = false, bool store = false) {
+  Dist t = make_raw_dist(a, ub * a.draws, a.K);
+  if (a.logits) {
+    float2 st;
+    if (first && a.K == 0) {
+      st = wave_row_stat(a, ub);
+      if (store && threadIdx.x == 0) a.rstat[ub] = st;
+    } else {
+      st = a.rstat[(long long)ub * a.rpb + a.K];
+    }
+    t.M = st.x;
+    t.invS = st.y;
+  }
   return t;
 }
 
-// Smallest kept probability of the top-p rule: the least v with
-// sum_{p_i > v} p_i <= top_p (fp64), found by bisection on the fp32 bits.
+// Smallest kept probability of group ub's bonus row t after select_kernel, in
+// mw_first_kernel (0: nothing is filtered).  All NT threads of the calling work-group.
 template <int NT>
-__device__ float topp_threshold(const Dist &t, int V, float top_p, double *red) {
-  uint32_t lo = 0, hi = 0x7f800000u;
-  while (hi - lo > 1) {
-    const uint32_t mid = lo + (hi - lo) / 2;
-    const float tau = u2f(mid);
-    double acc = 0.0;
-    for (int i = threadIdx.x; i < V; i += NT) {
-      const float p = t(i);
-      if (p > tau) acc += (double)p;
-    }
-    const double F = block_sum_f64<NT>(acc, red);
-    if (F <= (double)top_p)
-      hi = mid;
-    else
-      lo = mid;
-  }
-  return u2f(hi);
+__device__ float sel_finish(SelLds &L, const Args &a, int ub, const Dist &t) {
+  if (a.HG == 0) return 0.0f;
+  const SelRow r = a.sel[ub];
+  if (r.rules & kSelKnown) return u2f(r.C);
+  const int n = a.lcnt[ub];
+  const bool listed = n <= sel_cap(a);  // else more keys in one bin than the list holds: the row
+  return sel_levels<NT>(L, a, r.F, r.C, r.rules, r.bin, listed ? sel_list(a, ub) : nullptr, t,
+                        listed ? n : a.V);
 }
 
-// The top_k-th largest probability (ties kept): the least v with
-// #{p_i > v} < top_k, found by bisection on the fp32 bits.
-template <int NT>
-__device__ float topk_threshold(const Dist &t, int V, int top_k, double *red) {
-  uint32_t lo = 0, hi = 0x7f800000u;
-  while (hi - lo > 1) {
-    const uint32_t mid = lo + (hi - lo) / 2;
-    const float tau = u2f(mid);
-    double cnt = 0.0;
-    for (int i = threadIdx.x; i < V; i += NT) cnt += (t(i) > tau) ? 1.0 : 0.0;
-    if (block_sum_f64<NT>(cnt, red) < (double)top_k)
-      hi = mid;
-    else
-      lo = mid;
-  }
-  return u2f(hi);
-}
+// Whether the bonus rows are drawn from (python mode is in lock step).
+__device__ __forceinline__ bool sel_wanted(const Args &a) { return *a.nmin >= a.K - 1; }
 
-// ---------------------------------------------------------------------------
-// plan: the draw each sequence still needs.  Python mode applies the batch
-// lock-step rule n = min_b n_b of speculative.py:166 here; cpp mode's draws
-// are per sequence, so decide writes them directly.
-// ---------------------------------------------------------------------------
-
-// Python-mode draws take the first index whose sequential prefix sum
-// EXCEEDS u (so u = 0 never selects a zero-weight entry, as torch.multinomial
-// never does); the inverse-CDF walks test `r <= prefix`, and for floats
-// u < x <=> succ(u) <= x.  The floor FLT_MIN keeps r out of the denormals.
-__device__ __forceinline__ float py_threshold(float u) {
-  // for finite u >= 0 the next float up is the next bit pattern
-  const float s = (u >= 0.0f && u < INFINITY) ? __uint_as_float(__float_as_uint(u) + 1u) : u;
-  return fmaxf(s, 1.17549435e-38f);
-}
-
-// The job of sequence b: its draw (n, kind, row, eos_acc, threshold u; a
-// python-mode bonus after the resample when extra) and the statistics of the
-// draw's rows, once for every kernel that reads them.
-__device__ MwJob make_job(const Args &a, int b, int n, int kind, int row, int eos_acc, float u,
-                         int extra, float u2, const DecideLds *L) {
-  const int K = a.K;
-  MwJob j;
-  j.n = n;
-  j.kind = kind;
-  j.row = row;
-  j.eos_acc = eos_acc;
-  j.u = u;
-  j.extra = extra;
-  j.u2 = u2;
-  j.pad = 0;
-  j.tM = j.dM = 0.0f;
-  j.tInvS = j.dInvS = 1.0f;
-  if (a.logits && (j.kind == kResid || j.kind == kPlain)) {
-    // the rows' statistics, from the gather when it has them
-    const float2 ts = L ? L->st[j.row] : row_stat(a, (b / a.draws) * a.rpb + j.row);
-    j.tM = ts.x;
-    j.tInvS = ts.y;
-    if (j.kind == kResid) {
-      const float2 ds = L ? L->st[K + 1 + j.row] : row_stat(a, (b / a.draws) * a.rpb + K + 1 + j.row);
-      j.dM = ds.x;
-      j.dInvS = ds.y;
-    }
-  }
-  return j;
-}
-
-// Store the job and reset the walk state of b.
-__device__ void write_job(const Args &a, int b, const MwJob &j) {
-  a.jobs[b] = j;
-  a.res[b] = MwRes{0.0f, 0, -1, -1};
-  a.badcnt[b] = 0;
-  a.badcnt[a.B + b] = 0;
-}
-
-// Python mode only (cpp mode decides each sequence's draw by itself).
-__global__ __launch_bounds__(256) void plan_kernel(Args a) {
-  __shared__ int nmin;
-  const int K = a.K;
-  if (threadIdx.x == 0) nmin = K;
+// Grid (HG slices, groups): the bins of one slice of the bonus row.
+__global__ __launch_bounds__(kSelNT) void hist_kernel(Args a) {
+  __shared__ SelLds L;
+  const int ub = blockIdx.y, g = blockIdx.x;
+  if (g == 0 && threadIdx.x == 0) a.lcnt[ub] = 0;
+  if (!sel_wanted(a)) return;
+  const Dist t = sel_dist(a, ub, true, g == 0);
+  sel_zero<kSelNT>(L);
+  const bool sums = (sel_rules(a) & kRuleP) != 0;
+  sel_scan_row<kSelNT>(t, (long long)g * a.V / a.HG, (long long)(g + 1) * a.V / a.HG, sel_floor(a),
+                       [&](uint32_t key) { sel_add(L, sel_bin(key), key, sums); });
   __syncthreads();
-  int local = K;
-  for (int q = threadIdx.x; q < a.B; q += blockDim.x) local = min(local, a.dec[q].x);
-  atomicMin(&nmin, local);
-  __syncthreads();
-  // A rejection at the last position (n = K - 1) brings the reference's
-  // num_accepted to K, so its `num_accepted == self.k` branch
-  // (speculative.py:188-195) appends a bonus draw after the resample.
-  const int extra = (K > 0 && nmin == K - 1) ? 1 : 0;
-  for (int b = threadIdx.x; b < a.B; b += blockDim.x) {
-    const float u2 = extra ? py_threshold(a.U[(long long)b * a.ustride + K + 1]) : 0.0f;
-    write_job(a, b, make_job(a, b, nmin, (nmin < K) ? kResid : kPyBonus, (nmin < K) ? nmin : K, 0,
-                             py_threshold(a.ufin[b]), extra, u2));
+  double *hs = reinterpret_cast<double *>(sel_hist(a, ub) + (long long)g * kSelBytes);
+  uint32_t *hc = reinterpret_cast<uint32_t *>(hs + kSelBins);
+  for (int i = threadIdx.x; i < kSelBins; i += kSelNT) {
+    hs[i] = L.sum[i];
+    hc[i] = L.cnt[i];
   }
+}
+
+// Grid (HG slices, groups), after hist_kernel.
+__global__ __launch_bounds__(kSelNT) void select_kernel(Args a) {
+  __shared__ SelLds L;
+  __shared__ uint32_t keys[kSelMaxList];
+  __shared__ int nkeys, at;
+  const int ub = blockIdx.y, g = blockIdx.x;
+  if (!sel_wanted(a)) return;
+  const Dist t = sel_dist(a, ub);
+  int rules = sel_rules(a);
+  double F = 0.0;
+  uint32_t C = 0;
+  {
+    static_assert(kSelBins == kSelNT, "one bin per thread");
+    const unsigned char *h = sel_hist(a, ub);
+    double s = 0.0;
+    uint32_t c = 0;
+#pragma unroll 8
+    for (int q = 0; q < a.HG; ++q) {
+      const double *hs = reinterpret_cast<const double *>(h + (long long)q * kSelBytes);
+      s += hs[threadIdx.x];
+      c += reinterpret_cast<const uint32_t *>(hs + kSelBins)[threadIdx.x];
+    }
+    L.sum[threadIdx.x] = s;
+    L.cnt[threadIdx.x] = c;
+  }
+  if (threadIdx.x == 0) nkeys = 0;
+  __syncthreads();
+  const int bin = sel_find<kSelNT>(L, a, F, C, rules, false);
+  if (g == 0 && threadIdx.x == 0)
+    a.sel[ub] = bin < 0 ? SelRow{0.0, 1u, 0, kSelKnown}  // nothing cut: every positive probability
+                        : SelRow{F, C, (uint16_t)bin, (uint16_t)rules};
+  if (bin < 0) return;
+  const int cap = sel_cap(a);
+  sel_scan_row<kSelNT>(t, (long long)g * a.V / a.HG, (long long)(g + 1) * a.V / a.HG, sel_floor(a),
+                       [&](uint32_t key) {
+                         if (sel_bin(key) != bin) return;
+                         const int k = atomicAdd(&nkeys, 1);
+                         if (k < cap) keys[k] = key;
+                       });
+  __syncthreads();
+  const int n = nkeys;
+  if (threadIdx.x == 0) at = n ? atomicAdd(&a.lcnt[ub], n) : 0;
+  __syncthreads();
+  uint32_t *list = sel_list(a, ub);
+  for (int i = threadIdx.x; i < min(n, cap - at); i += kSelNT) list[at + i] = keys[i];
+}
+
+// Grid (groups): the whole selection of a short row.
+__global__ __launch_bounds__(kSelNT) void select_short_kernel(Args a) {
+  __shared__ SelLds L;
+  const int ub = blockIdx.x;
+  if (!sel_wanted(a)) return;
+  const Dist t = sel_dist(a, ub, true, true);
+  const float v = sel_levels<kSelNT>(L, a, 0.0, 0, sel_rules(a), -1, nullptr, t, a.V);
+  if (threadIdx.x == 0) a.sel[ub] = SelRow{0.0, f2u(v), 0, kSelKnown};
 }
 
 // ---------------------------------------------------------------------------
@@ -839,26 +1175,47 @@ __global__ __launch_bounds__(256) void plan_kernel(Args a) {
 enum MwPass : int { kPassSum = 0, kPassCdf = 1 };
 enum MwStatus : int { kChunkOk = 0, kChunkTiles = 1, kChunkSkipped = 2 };
 
-// The element function of a (job, pass): 0 max(0,t-d), 1 max(0,t-d)/S, 2 t.
+// The element function of a (job, pass): 0 max(0,t-d), 1 max(0,t-d)/S, 2 t,
+// and with KEEP (python mode and the filtered sampler) 3 the kept
+// probabilities (t >= vstar ? t : 0), 4 those / S.
+template <bool KEEP>
 struct MwElem {
   Dist t, d;
   int fn;
-  float S;
+  float S, vstar;
+  __device__ __forceinline__ bool reads_d() const { return fn < 2; }
   __device__ __forceinline__ float eval(float tv, float dv) const {
+    if (KEEP && fn > 2) {
+      const float p = t.eval(tv);
+      const float x = (p >= vstar) ? p : 0.0f;
+      return fn == 4 ? x / S : x;
+    }
     if (fn == 2) return t.eval(tv);
     const float x = relu_ref(t.eval(tv) - d.eval(dv));
     return fn == 1 ? x / S : x;
   }
 };
 
+// Draws whose elements are normalised by their exact sum first (two passes).
+template <bool KEEP>
+__device__ __forceinline__ bool mw_summed(const MwJob &j) {
+  return j.kind == kResid || (KEEP && j.kind == kPyBonus);
+}
+template <bool KEEP>
 __device__ __forceinline__ bool mw_active(const MwJob &j, int pass) {
-  return pass == kPassSum ? j.kind == kResid : (j.kind == kResid || j.kind == kPlain);
+  return mw_summed<KEEP>(j) || (pass == kPassCdf && j.kind == kPlain);
+}
+// A sum the second pass does not divide by: the residual then draws from t
+// (speculative.cpp:37), kept probabilities stay as they are.
+__device__ __forceinline__ int mw_fallback(const MwJob &j, float S) {
+  return j.kind == kResid ? (S <= 1e-6f ? 1 : 0) : (S > 0.0f ? 0 : 1);
 }
 
 // The element function of (job b, pass); `r` holds the sum pass's result
 // (S, fallback) for the CDF pass.
-__device__ __forceinline__ MwElem mw_elem_r(const Args &a, int b, const MwJob &j, int pass, const MwRes &r) {
-  MwElem e;
+template <bool KEEP>
+__device__ __forceinline__ MwElem<KEEP> mw_elem_r(const Args &a, int b, const MwJob &j, int pass, const MwRes &r) {
+  MwElem<KEEP> e;
   e.t.p = row_ptr(a, b, j.row);
   e.t.c = a.c;
   e.t.logits = a.logits;
@@ -866,6 +1223,12 @@ __device__ __forceinline__ MwElem mw_elem_r(const Args &a, int b, const MwJob &j
   e.t.invS = j.tInvS;
   e.d = e.t;
   e.S = 1.0f;
+  e.vstar = j.vstar;
+  if (KEEP && j.kind == kPyBonus) {
+    e.fn = (pass == kPassSum || r.fallback) ? 3 : 4;
+    e.S = r.S;
+    return e;
+  }
   if (j.kind == kResid) {
     e.d.p = row_ptr(a, b, a.K + 1 + j.row);
     e.d.M = j.dM;
@@ -880,17 +1243,22 @@ __device__ __forceinline__ MwElem mw_elem_r(const Args &a, int b, const MwJob &j
   return e;
 }
 
-__device__ __forceinline__ MwElem mw_elem(const Args &a, int b, const MwJob &j, int pass) {
-  return mw_elem_r(a, b, j, pass, pass == kPassSum ? MwRes{} : a.res[b]);
+template <bool KEEP>
+__device__ __forceinline__ MwElem<KEEP> mw_elem_sum(const Args &a, int b, const MwJob &j) {
+  return mw_elem_r<KEEP>(a, b, j, kPassSum, MwRes{});
 }
 
-// Raw values of 16 consecutive elements starting at i0 (zero past V).
+// Raw values of 16 consecutive elements starting at i0 (zero past V).  Four
+// 16-byte loads whatever the row's alignment: the hardware takes them at any
+// 4-byte boundary.
 __device__ __forceinline__ void mw_load16(const Args &a, const float *p, long long i0, float *v) {
-  if (a.vec && i0 + kMwTile <= a.V) {
-    const float4 *p4 = reinterpret_cast<const float4 *>(p + i0);
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  typedef f32x4 f32x4_u __attribute__((aligned(4)));
+  if (i0 + kMwTile <= a.V) {
+    const f32x4_u *p4 = reinterpret_cast<const f32x4_u *>(p + i0);
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      const float4 q = p4[k];
+      const f32x4 q = p4[k];
       v[4 * k] = q.x;
       v[4 * k + 1] = q.y;
       v[4 * k + 2] = q.z;
@@ -904,23 +1272,26 @@ __device__ __forceinline__ void mw_load16(const Args &a, const float *p, long lo
 
 // Raw target and draft values of tile `tile` (the draft only when the
 // element function reads it).
-__device__ __forceinline__ void mw_tile_raw(const Args &a, const MwElem &e, long long tile,
+template <class E>
+__device__ __forceinline__ void mw_tile_raw(const Args &a, const E &e, long long tile,
                                             float *tv, float *dv) {
   const long long i0 = tile * kMwTile;
   mw_load16(a, e.t.p, i0, tv);
-  if (e.fn != 2) mw_load16(a, e.d.p, i0, dv);
+  if (e.reads_d()) mw_load16(a, e.d.p, i0, dv);
 }
 
 // Evaluated elements of tile `tile` from its raw values (zero past V).
-__device__ __forceinline__ void mw_tile_eval(const Args &a, const MwElem &e, long long tile,
+template <class E>
+__device__ __forceinline__ void mw_tile_eval(const Args &a, const E &e, long long tile,
                                              const float *tv, const float *dv, float *x) {
   const long long i0 = tile * kMwTile;
 #pragma unroll
-  for (int k = 0; k < kMwTile; ++k) x[k] = (i0 + k < a.V) ? e.eval(tv[k], e.fn != 2 ? dv[k] : 0.0f) : 0.0f;
+  for (int k = 0; k < kMwTile; ++k) x[k] = (i0 + k < a.V) ? e.eval(tv[k], e.reads_d() ? dv[k] : 0.0f) : 0.0f;
 }
 
 // Evaluated elements of tile `tile` of a row (zero past V).
-__device__ __forceinline__ void mw_tile_values(const Args &a, const MwElem &e, long long tile,
+template <class E>
+__device__ __forceinline__ void mw_tile_values(const Args &a, const E &e, long long tile,
                                                float *x) {
   float tv[kMwTile], dv[kMwTile];
   mw_tile_raw(a, e, tile, tv, dv);
@@ -1086,7 +1457,7 @@ __device__ __forceinline__ void mw_records_chunk(const Args &a, int b, int c, in
 
 // Zeroes this work-group's share (work-group wg of nwg) of the first exact
 // pass's look-back words, of both passes' cache counters and of the tail
-// kernel's synchronisation words.  The first kernel of every call that draws
+// kernel's synchronisation words; python mode's accept count starts at K.  The first kernel of every call that draws
 // exactly runs this, so nothing in the workspace has to start at zero.
 __device__ void mw_reset_share(const Args &a, long long wg, long long nwg) {
   const long long nt = blockDim.x, i0 = wg * nt + threadIdx.x, step = nwg * nt;
@@ -1095,6 +1466,7 @@ __device__ void mw_reset_share(const Args &a, long long wg, long long nwg) {
     a.badcnt[i] = 0;
     a.tsync[i] = 0ull;
   }
+  if (a.nmin != nullptr && i0 == 0) *a.nmin = a.K;
 }
 
 __global__ __launch_bounds__(256) void mw_reset_kernel(Args a) {
@@ -1265,7 +1637,9 @@ constexpr int kMwChunksPerWG = (kMwNT / 64) * kMwCPW;
 // c0 + 1 (c0 = 2 (4 blockIdx.x + wave)) of job blockIdx.y, lane = tile in the
 // chunk.  With `decide` (cpp rules) every work-group first takes sequence
 // b's decision itself (decide_cpp: the same inputs, so the same job
-// everywhere) and the first one stores it.  Every active job stores its
+// everywhere), otherwise it forms the job from py_decide_kernel's results
+// (and finishes the selection of a bonus row's smallest kept probability);
+// the first one stores the job.  Every active job stores its
 // chunk sums of t (the CDF pass of a plain draw, or of the fallback, starts
 // from them); a residual job also stores those of max(0, t - d), finds its
 // chunks' entry values by look-back (both chunks' own sums published first),
@@ -1273,6 +1647,7 @@ constexpr int kMwChunksPerWG = (kMwNT / 64) * kMwCPW;
 // chunk 0 then walks it (the walk's slowest chunk: its small running value
 // crosses a binade every few elements) and stores the exact running value
 // after it, so the sum pass's walk starts at chunk 1.
+template <bool KEEP>
 __global__ __launch_bounds__(kMwNT) void mw_first_kernel(Args a, int decide) {
   __shared__ __align__(16) float xs0[kMwChunk];  // chunk 0's values and tile records
   __shared__ MwRec tr0[kMwChunkTiles];
@@ -1288,27 +1663,35 @@ __global__ __launch_bounds__(kMwNT) void mw_first_kernel(Args a, int decide) {
       sj = decide_cpp(a, b, L);
       if (blockIdx.x == 0) {  // the cache counters were zeroed by an earlier kernel
         a.jobs[b] = sj;
-        a.res[b] = MwRes{0.0f, 0, -1, -1};
+        a.res[b] = MwRes{0.0f, 0, -1, 0};
       }
     }
     __syncthreads();
     j = sj;
   } else {
-    j = a.jobs[b];
+    j = py_job(a, b);
   }
-  if (j.kind != kResid && j.kind != kPlain) return;
-  if (c0 >= a.NC) return;
+  if (!mw_active<KEEP>(j, kPassCdf)) return;
   const bool two = c0 + 1 < a.NC;
-  const bool resid = j.kind == kResid;
-  const MwElem e = mw_elem(a, b, j, kPassSum);
+  const bool resid = j.kind == kResid, summed = mw_summed<KEEP>(j);
+  MwElem<KEEP> e = mw_elem_sum<KEEP>(a, b, j);
   float tv[kMwCPW][kMwTile], dv[kMwCPW][kMwTile], x[kMwCPW][kMwTile];
-  // both chunks' loads before any use
+  // both chunks' loads before any use (and before the selection)
 #pragma unroll
   for (int h = 0; h < kMwCPW; ++h) {
-    const long long i0 = ((long long)(c0 + (two ? h : 0)) * kMwChunkTiles + lane) * kMwTile;
+    const long long i0 = ((long long)min(c0 + (two ? h : 0), a.NC - 1) * kMwChunkTiles + lane) * kMwTile;
     mw_load16(a, e.t.p, i0, tv[h]);
     if (resid) mw_load16(a, e.d.p, i0, dv[h]);
   }
+  if constexpr (KEEP) {
+    // (the bonus after a resample too: mw_tail_kernel writes over the lists)
+    if (j.kind == kPyBonus || (j.extra && blockIdx.x == 0)) {
+      __shared__ SelLds SL;
+      j.vstar = e.vstar = sel_finish<kMwNT>(SL, a, b / a.draws, sel_dist(a, b / a.draws));
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) a.jobs[b] = j;  // for the kernels after this one
+  }
+  if (c0 >= a.NC) return;
   float sx[kMwCPW];
 #pragma unroll
   for (int h = 0; h < kMwCPW; ++h) {
@@ -1323,6 +1706,9 @@ __global__ __launch_bounds__(kMwNT) void mw_first_kernel(Args a, int decide) {
         if (resid) {
           x[h][k] = relu_ref(tp - e.d.eval(dv[h][k]));
           sxh += x[h][k];
+        } else if (KEEP && summed) {
+          x[h][k] = (tp >= e.vstar) ? tp : 0.0f;
+          sxh += x[h][k];
         }
       }
     }
@@ -1333,7 +1719,7 @@ __global__ __launch_bounds__(kMwNT) void mw_first_kernel(Args a, int decide) {
       a.csum_x[(long long)b * a.NC + c0 + h] = sx[h];
     }
   }
-  if (!resid) return;
+  if (!summed) return;
   unsigned long long *fl = a.flags + (long long)b * a.NC;
   if (two && lane == 0) lb_store(fl + c0 + 1, kLbAgg | f2u(sx[1]));  // before c0's look-back
   const float E0 = mw_lookback(a, b, c0, sx[0]);
@@ -1359,12 +1745,13 @@ __device__ __forceinline__ void finish_one(const Args &a, int b, const MwJob &j,
 
 // Last index of positive weight of a (job, pass) row, V - 1 if none; one
 // wave scans down from the end (python mode's rare fallback draw).
-__device__ long long mw_last_positive(const Args &a, const MwElem &e) {
+template <class E>
+__device__ long long mw_last_positive(const Args &a, const E &e) {
   const int lane = threadIdx.x & 63;
   for (long long base = ((long long)(a.V - 1) / 64) * 64; base >= 0; base -= 64) {
     const long long i = base + lane;
     bool pos = false;
-    if (i < a.V) pos = e.eval(e.t.load(i), e.fn != 2 ? e.d.load(i) : 0.0f) > 0.0f;
+    if (i < a.V) pos = e.eval(e.t.load(i), e.reads_d() ? e.d.load(i) : 0.0f) > 0.0f;
     const unsigned long long m = __ballot(pos);
     if (m) return base + 63 - __builtin_clzll(m);
   }
@@ -1384,13 +1771,14 @@ struct MwWalkLds {
 // The exact walk of job b's row for one pass, by the calling wave alone: it
 // synchronises only itself, so the other waves of its work-group can wait at
 // a barrier meanwhile.  Writes the pass's result (sum pass: S and the
-// fallback flag; CDF pass: the drawn index, and the outputs in cpp mode) and
+// fallback flag; CDF pass: the drawn index, and the outputs) and
 // returns the final running value.  use_cache = false ignores the cached
 // serial tiles (another work-group may still be filling a slot); the walk
 // then reads those tiles' values from the row.  pre0: chunk 0 was already
 // walked (mw_walk_chunk0), ending at running value s0 with hit found0.
+template <class E>
 __device__ __forceinline__ float mw_walk(const Args &a, int b, int pass, const MwJob &j,
-                                         const MwElem &e, MwWalkLds &L, bool use_cache = true,
+                                         const E &e, MwWalkLds &L, bool use_cache = true,
                                          bool pre0 = false, float s0 = 0.0f, long long found0 = -1) {
   using namespace seq;
   MwChunk *cr = L.cr;
@@ -1553,21 +1941,18 @@ __device__ __forceinline__ float mw_walk(const Args &a, int b, int pass, const M
     };
     found = walk(cnt, s, cdf, r, chunk_item, chunk_desc);
   }
+  // Python mode: past the end of the prefix sums, the last entry of
+  // positive weight (the reference's C++ rule, V - 1, is kept in cpp mode).
+  if (cdf && a.mode == CFA_MODE_PYTHON && found < 0) found = mw_last_positive(a, e);
   if (lane == 0) {
     if (!cdf) {
       a.res[b].S = s;
-      a.res[b].fallback = (s <= 1e-6f) ? 1 : 0;  // speculative.cpp:37
+      a.res[b].fallback = mw_fallback(j, s);
     } else {
       const int idx = (found < 0 || found >= a.V) ? a.V - 1 : (int)found;
       a.res[b].idx = idx;
-      if (a.mode == CFA_MODE_CPP) finish_one(a, b, j, idx);
+      if (!j.extra) finish_one(a, b, j, idx);  // else pybonus_kernel does
     }
-  }
-  // Python mode: past the end of the prefix sums, the last entry of
-  // positive weight (the reference's C++ rule, V - 1, is kept in cpp mode).
-  if (cdf && a.mode == CFA_MODE_PYTHON && found < 0) {
-    const long long last = mw_last_positive(a, e);
-    if (lane == 0) a.res[b].idx = (int)last;
   }
   return s;
 }
@@ -1617,6 +2002,7 @@ __device__ __forceinline__ void mw_tail_ids(int L, int &b, int &part) {
   part = w / 8;
 }
 
+template <bool KEEP>
 __global__ __launch_bounds__(kMwTailNT) void mw_tail_kernel(Args a) {
   __shared__ MwWalkLds L;
   __shared__ float Es[kMwMaxNC];  // approximate chunk entry values (before the 1 / S)
@@ -1627,14 +2013,14 @@ __global__ __launch_bounds__(kMwTailNT) void mw_tail_kernel(Args a) {
   if (b >= a.B) return;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const MwJob j = a.jobs[b];
-  if (!mw_active(j, kPassCdf)) {
+  if (!mw_active<KEEP>(j, kPassCdf)) {
     if (part == 0 && a.mode == CFA_MODE_CPP && threadIdx.x == 0) finish_one(a, b, j, -1);
     return;
   }
-  const bool resid = j.kind == kResid;
+  const bool resid = j.kind == kResid, summed = mw_summed<KEEP>(j);
   // a wave that does not walk scans the chunk sums of the CDF pass's row
   if (wave == 1) {
-    const float *csum = (resid ? a.csum_x : a.csum_t) + (long long)b * a.NC;
+    const float *csum = (summed ? a.csum_x : a.csum_t) + (long long)b * a.NC;
     float carry = 0.0f;
     for (int base = 0; base < a.NC; base += 64) {
       const float v = (base + lane < a.NC) ? csum[base + lane] : 0.0f;
@@ -1644,12 +2030,12 @@ __global__ __launch_bounds__(kMwTailNT) void mw_tail_kernel(Args a) {
     }
   }
   unsigned long long *ts = a.tsync + 2LL * b;
-  MwRes r{0.0f, 0, -1, -1};
-  if (resid) {
+  MwRes r{0.0f, 0, -1, 0};
+  if (summed) {
     if (part == 0) {
       if (wave == 0) {
         // chunk 0 was walked by the first pass (a.s0)
-        const float S = mw_walk(a, b, kPassSum, j, mw_elem(a, b, j, kPassSum), L, true, true, a.s0[b]);
+        const float S = mw_walk(a, b, kPassSum, j, mw_elem_sum<KEEP>(a, b, j), L, true, true, a.s0[b]);
         if (lane == 0) {
           sS = S;
           __hip_atomic_store(ts, kTsyncSet | f2u(S), __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
@@ -1669,16 +2055,16 @@ __global__ __launch_bounds__(kMwTailNT) void mw_tail_kernel(Args a) {
     __syncthreads();
     if (part != 0 && !sok) return;  // the walker writes this part's share
     r.S = sS;
-    r.fallback = (r.S <= 1e-6f) ? 1 : 0;  // speculative.cpp:37, as the walk stores it
+    r.fallback = mw_fallback(j, r.S);
   } else {
     __syncthreads();  // Es
   }
-  const MwElem e = mw_elem_r(a, b, j, kPassCdf, r);
+  const MwElem<KEEP> e = mw_elem_r<KEEP>(a, b, j, kPassCdf, r);
   // approximate entry value of chunk c on the CDF pass's scale (a residual
   // job whose sum fell to the fallback draws from t: t's own chunk sums)
   auto entry = [&](int c) __attribute__((always_inline)) -> float {
     if (resid && e.fn == 2) return mw_entry_prefix(a.csum_t + (long long)b * a.NC, c);
-    return (e.fn == 1) ? Es[c] / e.S : Es[c];
+    return (e.fn == 1 || (KEEP && e.fn == 4)) ? Es[c] / e.S : Es[c];
   };
   // records of chunk c; a chunk surely past u gets a "skipped" record and no
   // loads.  Chunk 0 (never skipped: its entry value is 0) also goes to the
@@ -1740,8 +2126,9 @@ __global__ __launch_bounds__(kMwTailNT) void mw_tail_kernel(Args a) {
 }
 
 // ---------------------------------------------------------------------------
-// python-mode bonus draw (top-p filter, renormalise, draw; speculative.py:
-// 65-84): one work-group per sequence with the block-level exact replay.
+// python mode: the bonus that follows a resample at the last draft position
+// (speculative.py:188-195), a second draw of the same sequence: one
+// work-group per sequence with the block-level exact replay.
 // ---------------------------------------------------------------------------
 
 constexpr int kSampleNT = 1024;
@@ -1765,17 +2152,14 @@ __device__ long long block_last_positive(const XF &xf, int V, int *slot) {
 
 __global__ __launch_bounds__(kSampleNT) void pybonus_kernel(Args a) {
   __shared__ seq::Shared<kSampleNT> sh;
-  __shared__ double red[kSampleNT / 64];
   __shared__ int last;
   const int b = blockIdx.x, V = a.V;
   const MwJob j = a.jobs[b];
-  // the bonus of a full acceptance, or the one after a rejection at K - 1
-  if (j.kind != kPyBonus && !j.extra) return;
-  const float u = (j.kind == kPyBonus) ? j.u : j.u2;
-  const Dist t = make_dist(a, b, a.K);
+  if (!j.extra) return;
+  const float u = j.u2;
+  const Dist t = sel_dist(a, b / a.draws);
   long long idx = -1;
-  float vstar = (a.top_p < 1.0f) ? topp_threshold<kSampleNT>(t, V, a.top_p, red) : 0.0f;
-  if (a.top_k > 0 && a.top_k < V) vstar = fmaxf(vstar, topk_threshold<kSampleNT>(t, V, a.top_k, red));
+  const float vstar = j.vstar;
   const float S = seq::run<kSampleNT>(XKeep{t, vstar}, V, false, 0.0f, sh, nullptr);
   if (S > 0.0f) {
     const XKeepNorm xf{t, vstar, S};
@@ -1786,12 +2170,7 @@ __global__ __launch_bounds__(kSampleNT) void pybonus_kernel(Args a) {
     seq::run<kSampleNT>(xf, V, true, u, sh, &idx);
     if (idx < 0) idx = block_last_positive<kSampleNT>(xf, V, &last);
   }
-  if (threadIdx.x == 0) {
-    if (j.kind == kPyBonus)
-      a.res[b].idx = (int)idx;
-    else
-      a.res[b].idx2 = (int)idx;
-  }
+  if (threadIdx.x == 0) finish_one(a, b, j, a.res[b].idx, (int)idx);
 }
 
 // ---------------------------------------------------------------------------
@@ -1819,15 +2198,6 @@ __device__ __forceinline__ void finish_one(const Args &a, int b, const MwJob &j,
   a.out_final[b] = fin;
   a.out_eos[b] = (a.mode == CFA_MODE_CPP) ? ((eos_acc || fin == a.eos) ? 1 : 0) : 0;
   a.out_num_emitted[b] = eos_acc ? n : n + 1 + (j.extra ? 1 : 0);
-}
-
-// Python mode (cpp mode finishes each sequence at the end of its last walk).
-__global__ __launch_bounds__(64) void finish_kernel(Args a) {
-  const int b = blockIdx.x * 64 + threadIdx.x;
-  if (b >= a.B) return;
-  const MwJob j = a.jobs[b];
-  const MwRes r = a.res[b];
-  finish_one(a, b, j, r.idx, r.idx2);
 }
 
 // Optional: write the probabilities the verification used.
@@ -1968,14 +2338,31 @@ static int stats_slices(long long R, long long Vw) {
   const long long by_rows = std::min<long long>((1024 + R - 1) / R, std::max<long long>(1, Vw / 256));
   return (int)std::min<long long>(256, std::max<long long>(1, std::max(by_len, by_rows)));
 }
+// Histogram slices per row of the kept-probability selection: about 512
+// work-groups in all, each with room for its bins; 1 (select_short_kernel)
+// for rows without room for two, 0 when nothing is filtered.
+static int sel_slices(const Args &a, int groups) {
+  if (!(a.top_p < 1.0f) && !(a.top_k > 0 && a.top_k < a.V)) return 0;
+  if (a.NC < kSelMinNC) return 1;
+  const int room = a.NC * kMwChunkTiles * (int)sizeof(MwRec) / kSelBytes;
+  return std::max(2, std::min({kSelMaxHG, room, (512 + groups - 1) / groups}));
+}
 // Head positions of the two-pass statistics (cpp rules, logits): with the
 // ~0.7 per-position acceptance of typical draft models, 3 minimises the rows
 // the two passes read together.
 constexpr int kHeadPositions = 3;
+// Python mode's lock step stops a batch of B at a position with probability
+// 1 - 0.7^B, so one head position is enough.
+constexpr int kPyHeadPositions = 1;
+// Below this many bytes of rows one pass over all of them is faster: the
+// second launch waits for the first and then for each row's partials, of
+// which few rows have many (B = 8, K = 5, V = 128256, 45 MB, cpp rules:
+// 67.8 us in one pass, 85 in two; B = 64, 361 MB: 140 against 124).
+constexpr long long kTwoPassBytes = 128ll << 20;
 
 // Workspace layout (each region 256-byte aligned).
 struct WsLayout {
-  size_t part, apart, rawtok, dec, ufin, jobs, res, csum_x, csum_t, crec, trec, badcnt, bad, x0, flags,
+  size_t part, apart, rawtok, sel, lcnt, jobs, res, csum_x, csum_t, crec, trec, badcnt, bad, x0, flags,
       tsync, s0, total;
 };
 
@@ -1995,8 +2382,8 @@ static WsLayout ws_layout(int B, int K, int V, int mode) {
   L.part = take(G * sizeof(float2));
   L.apart = take(G * sizeof(float2));
   L.rawtok = take(R * sizeof(float));
-  L.dec = take((size_t)B * sizeof(int4));
-  L.ufin = take((size_t)B * sizeof(float));
+  L.sel = take((size_t)B * sizeof(SelRow));
+  L.lcnt = take((size_t)B * sizeof(int));
   L.jobs = take((size_t)B * sizeof(MwJob));
   L.res = take((size_t)B * sizeof(MwRes));
   L.csum_x = take(mw ? (size_t)B * NC * sizeof(float) : 0);
@@ -2100,22 +2487,21 @@ static int run_pipeline(Args &a, bool vec, void *workspace, hipStream_t st, floa
   const int R = (B / a.draws) * a.rpb;
   a.R = R;
   a.S = stats_slices(R, a.Vw);
-  // cpp rules with logits: statistics in two passes, the second only for the
-  // sequences that accepted every head position (not when the caller asks
-  // for every row's probabilities)
-  const bool two_pass = mode == CFA_MODE_CPP && a.logits && a.draws == 1 && K > kHeadPositions &&
+  // statistics in two passes, the second only for the sequences that
+  // accepted every head position (not when the caller asks for every row's
+  // probabilities)
+  const int head = mode == CFA_MODE_PYTHON ? kPyHeadPositions : kHeadPositions;
+  const bool two_pass = (mode == CFA_MODE_CPP || (mode == CFA_MODE_PYTHON && R / a.rpb <= kTailMaxGroups)) &&
+                        K > head && (long long)R * V * 4 >= kTwoPassBytes && a.logits && a.draws == 1 &&
                         !out_target_probs && !out_draft_probs;
-  a.P = two_pass ? kHeadPositions : K;
+  a.P = two_pass ? head : K;
 
-  a.vec = vec ? 1 : 0;
   a.NC = (V + kMwChunk - 1) / kMwChunk;
   const WsLayout L = ws_layout(B, K, V, mode);
   char *ws = (char *)workspace;
   a.part = (float2 *)(ws + L.part);
   a.apart = (float2 *)(ws + L.apart);
   a.rawtok = (float *)(ws + L.rawtok);
-  a.dec = (int4 *)(ws + L.dec);
-  a.ufin = (float *)(ws + L.ufin);
   a.jobs = (MwJob *)(ws + L.jobs);
   a.res = (MwRes *)(ws + L.res);
   a.csum_x = (float *)(ws + L.csum_x);
@@ -2128,6 +2514,11 @@ static int run_pipeline(Args &a, bool vec, void *workspace, hipStream_t st, floa
   a.flags = (unsigned long long *)(ws + L.flags);
   a.tsync = (unsigned long long *)(ws + L.tsync);
   a.s0 = (float *)(ws + L.s0);
+  a.sel = (SelRow *)(ws + L.sel);
+  a.lcnt = (int *)(ws + L.lcnt);
+  a.rstat = a.apart;  // the argmax partials' room: greedy mode only
+  a.nmin = mode == CFA_MODE_PYTHON ? &a.res[0].nmin : nullptr;
+  a.HG = mode == CFA_MODE_PYTHON ? sel_slices(a, R / a.rpb) : 0;
   // the first statistics pass zeroes the look-back words, cache counters and
   // tail synchronisation words; without one (probabilities input) a small
   // kernel does
@@ -2153,10 +2544,13 @@ static int run_pipeline(Args &a, bool vec, void *workspace, hipStream_t st, floa
     int rc;
     if (two_pass) {
       if ((rc = stats(kRowsHead, groups * 2 * a.P)) != CFA_OK) return rc;
-      if (vec && groups <= kTailMaxGroups) {
+      if (groups <= kTailMaxGroups) {
         const long long items = (long long)groups * (2 * (K - a.P) + 1) * a.S;
         const int grid = (int)std::min<long long>(items, (long long)kTailPerCU * device_cu_count());
-        CFA_LAUNCH("chain_stats_tail", stats_tail_kernel<kStatsNT>, dim3(grid), dim3(kStatsNT), 0, st, a);
+        if (vec)
+          CFA_LAUNCH("chain_stats_tail", (stats_tail_kernel<kStatsNT, 4>), dim3(grid), dim3(kStatsNT), 0, st, a);
+        else
+          CFA_LAUNCH("chain_stats_tail", (stats_tail_kernel<kStatsNT, 1>), dim3(grid), dim3(kStatsNT), 0, st, a);
       } else if ((rc = stats(kRowsTail, groups * (2 * (K - a.P) + 1))) != CFA_OK) {
         return rc;
       }
@@ -2167,19 +2561,27 @@ static int run_pipeline(Args &a, bool vec, void *workspace, hipStream_t st, floa
   if (mode == CFA_MODE_GREEDY)
     CFA_LAUNCH("chain_argmax", (argmax_kernel<256>), dim3((unsigned)R, (unsigned)a.S), dim3(256), 0,
                st, a);
-  // cpp rules: the mw sums kernel takes each sequence's decision itself
-  const int fused_decide = mode == CFA_MODE_CPP ? 1 : 0;
-  if (!fused_decide) CFA_LAUNCH("chain_decide", decide_kernel, dim3(B), dim3(64), 0, st, a);
+  // (cpp rules: mw_first_kernel takes each sequence's decision itself)
+  if (mode == CFA_MODE_GREEDY) CFA_LAUNCH("chain_decide", decide_kernel, dim3(B), dim3(64), 0, st, a);
   if (mode != CFA_MODE_GREEDY) {
     const dim3 cg1((a.NC + kMwChunksPerWG - 1) / kMwChunksPerWG, B);   // two chunks per wave
     const unsigned tail_wgs = (unsigned)(((B + 7) / 8) * 8 * kMwTailWGs);
-    if (mode == CFA_MODE_PYTHON) CFA_LAUNCH("chain_plan", plan_kernel, dim3(1), dim3(256), 0, st, a);
-    CFA_LAUNCH("chain_mw_first", mw_first_kernel, cg1, dim3(kMwNT), 0, st, a, fused_decide);
-    CFA_LAUNCH("chain_mw_tail", mw_tail_kernel, dim3(tail_wgs), dim3(kMwTailNT), 0, st, a);
-    if (mode == CFA_MODE_PYTHON)
-      CFA_LAUNCH("chain_pybonus", pybonus_kernel, dim3(B), dim3(kSampleNT), 0, st, a);
-    if (mode == CFA_MODE_PYTHON)
-      CFA_LAUNCH("chain_finish", finish_kernel, dim3((B + 63) / 64), dim3(64), 0, st, a);
+    if (mode == CFA_MODE_PYTHON) {
+      if (K > 0 || a.HG == 0)
+        CFA_LAUNCH("chain_decide", py_decide_kernel, dim3(R / a.rpb), dim3(64 * std::min(a.rpb, 16)), 0, st, a);
+      if (a.HG > 1) {
+        CFA_LAUNCH("chain_hist", hist_kernel, dim3(a.HG, R / a.rpb), dim3(kSelNT), 0, st, a);
+        CFA_LAUNCH("chain_select", select_kernel, dim3(a.HG, R / a.rpb), dim3(kSelNT), 0, st, a);
+      } else if (a.HG == 1) {
+        CFA_LAUNCH("chain_select", select_short_kernel, dim3(R / a.rpb), dim3(kSelNT), 0, st, a);
+      }
+      CFA_LAUNCH("chain_mw_first", mw_first_kernel<true>, cg1, dim3(kMwNT), 0, st, a, 0);
+      CFA_LAUNCH("chain_mw_tail", mw_tail_kernel<true>, dim3(tail_wgs), dim3(kMwTailNT), 0, st, a);
+      if (K > 0) CFA_LAUNCH("chain_pybonus", pybonus_kernel, dim3(B), dim3(kSampleNT), 0, st, a);
+    } else {
+      CFA_LAUNCH("chain_mw_first", mw_first_kernel<false>, cg1, dim3(kMwNT), 0, st, a, 1);
+      CFA_LAUNCH("chain_mw_tail", mw_tail_kernel<false>, dim3(tail_wgs), dim3(kMwTailNT), 0, st, a);
+    }
   }
   if (out_target_probs || out_draft_probs) {
     const int gx = std::min(64, (V + 255) / 256);

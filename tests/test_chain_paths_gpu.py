@@ -1,0 +1,70 @@
+"""GPU tier: the routes chain verification takes by shape, each against the
+oracle fed the probabilities the kernel used: many statistics slices per row
+(few rows), rows at every 4-byte alignment, and python mode's two-pass
+statistics (a large batch), whose second pass is read by the whole batch or
+by no one."""
+import numpy as np
+import pytest
+import torch
+
+from cudaforge_amd.verify import chain_verify
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _inputs(B, K, V, seed, device):
+    g = torch.Generator(device=device).manual_seed(seed)
+    tl = 2.0 * torch.randn(B, K + 1, V, device=device, generator=g)
+    dl = (tl[:, :K] + 0.5 * torch.randn(B, K, V, device=device, generator=g)).contiguous()
+    tok = torch.multinomial(torch.softmax(dl, -1).view(B * K, V), 1, generator=g).view(B, K).int()
+    return tl, dl, tok, torch.rand(B, K + 2, device=device, generator=g)
+
+
+def _want(mode, tp, dp, tok, u, top_p):
+    if mode == "cpp":
+        w = O.chain_verify(tp, dp, tok, u)
+        return w["accept_len"], w["tokens"]
+    n, _, toks = O.python_verify(tp, dp, tok, u, top_p)
+    return n, toks
+
+
+@pytest.mark.parametrize("mode", ["cpp", "python"])
+@pytest.mark.parametrize("B,K,V", [(1, 4, 32000), (1, 8, 128256), (2, 3, 20001), (3, 2, 20002),
+                                   (2, 5, 40003), (5, 1, 999)])
+@pytest.mark.parametrize("accept", [False, True])
+def test_few_rows(device, mode, B, K, V, accept):
+    tl, dl, tok, u = _inputs(B, K, V, B * V + K, device)
+    if accept:
+        u[:, :K] = 0.0                      # every draft accepted: the bonus row is drawn from
+    u = u[:, : K + 1].contiguous() if mode == "cpp" else u
+    o = chain_verify(tl, dl, tok, u, mode=mode, top_p=0.9, return_probs=True)
+    plain = chain_verify(tl, dl, tok, u, mode=mode, top_p=0.9)
+    n, toks = _want(mode, o.target_probs.cpu().numpy(), o.draft_probs.cpu().numpy(),
+                    tok.cpu().numpy(), u.cpu().numpy(), 0.9)
+    assert np.array_equal(o.accept_len.cpu().numpy().ravel(), np.broadcast_to(n, (B,)))
+    assert np.array_equal(o.tokens.cpu().numpy(), toks)
+    assert torch.equal(plain.tokens, o.tokens) and torch.equal(plain.final, o.final)
+
+
+@pytest.mark.parametrize("V", [33000, 33001])
+@pytest.mark.parametrize("case", ["reject", "accept", "last"])
+def test_python_two_pass(device, V, case):
+    """143 MB of rows; return_probs forces one pass over all of them.  "last":
+    the batch's first rejection is at K - 1, so a bonus follows the resample."""
+    B, K = 64, 8
+    tl, dl, tok, u = _inputs(B, K, V, V, device)
+    if case != "reject":
+        u[:, :K] = 0.0
+    if case == "last":
+        u[7, K - 1] = 1.0 - 2.0 ** -24
+        tl[7, K - 1, tok[7, K - 1].long()] -= 6.0
+    a = chain_verify(tl, dl, tok, u, mode="python", top_p=0.9)
+    o = chain_verify(tl, dl, tok, u, mode="python", top_p=0.9, return_probs=True)
+    for x, y in ((a.tokens, o.tokens), (a.accept_len, o.accept_len), (a.final, o.final),
+                 (a.num_emitted, o.num_emitted)):
+        assert torch.equal(x, y)
+    n, toks = _want("python", o.target_probs.cpu().numpy(), o.draft_probs.cpu().numpy(),
+                    tok.cpu().numpy(), u.cpu().numpy(), 0.9)
+    assert np.array_equal(a.tokens.cpu().numpy(), toks)
+    assert {"accept": K, "last": K - 1}.get(case, int(a.accept_len[0])) == int(a.accept_len[0])
