@@ -1,0 +1,25 @@
+// w4a16_few.hpp -- host interface of the few-row W4A16 GEMM (w4a16_few.hip),
+// to which the entry points of w4a16_gemm.hip route small M.
+#pragma once
+
+#include <stdint.h>
+
+namespace cfa {
+namespace w4few {
+
+constexpr int kMaxM = 128;
+
+// Splits of K for a shape (N % 128 == 0, K % 128 == 0).
+int splits(int M, int N, int K);
+
+// form: how the weights are formed (0 bf16 as cfa_w4a16_dequant, 1 bf16 as
+// cfa_w4a16_gemm_zp, 2 fp16).  out: 0 C [M, N], 1 SiLU-gated C [M, N / 2] (S == 1), 2 fp32 partials
+// part [S, M, N].  The caller has checked shapes and 16-byte alignment.
+int launch(const void *a, const uint32_t *b_quant, const void *scales, const void *zeros, int M, int N, int K,
+           int group, int form, void *c, float *part, int S, int out, void *stream);
+
+// c [MN] fp16 = the partials' sum in split order
+int reduce_f16(const float *part, void *c, long long MN, int S, void *stream);
+
+}  // namespace w4few
+}  // namespace cfa

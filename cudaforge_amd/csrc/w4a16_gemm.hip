@@ -34,6 +34,7 @@
 #include "abi_internal.hpp"
 #include "lds_dma.hpp"
 #include "silu.hpp"
+#include "w4a16_few.hpp"
 
 namespace cfa {
 namespace w4mm {
@@ -414,6 +415,9 @@ __global__ __launch_bounds__(256) void w4mm_reduce_silu_kernel(const float *part
   *reinterpret_cast<uint2 *>(C + i) = o;
 }
 
+// Shapes the few-row kernel (w4a16_few.hip) takes.
+inline bool few_rows(int M, int N, int K) { return M <= w4few::kMaxM && N % 128 == 0 && K % 128 == 0; }
+
 // Splits of K: enough work-groups for every CU, each split at least 8
 // slices; *spp slices per split, and no split empty.
 int choose_splits(int M, int N, int K, int cus, int *spp) {
@@ -426,13 +430,55 @@ int choose_splits(int M, int N, int K, int cus, int *spp) {
   return (nsl + per - 1) / per;
 }
 
+// The splits an entry point uses: those of the few-row kernel or of this one.
+int splits_of(int M, int N, int K) {
+  return few_rows(M, N, K) ? w4few::splits(M, N, K) : choose_splits(M, N, K, abi::device_cu_count(), nullptr);
+}
+
 }  // namespace w4mm
 }  // namespace cfa
 
 extern "C" size_t cfa_w4a16_gemm_zp_workspace_size(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0 || N % cfa::w4mm::kBN != 0 || K % cfa::w4mm::kSK != 0) return 0;
-  const int s = cfa::w4mm::choose_splits(M, N, K, cfa::abi::device_cu_count(), nullptr);
+  const int s = cfa::w4mm::splits_of(M, N, K);
   return s > 1 ? (size_t)s * M * N * sizeof(float) : 0;
+}
+
+// The sum of the split partials into c: bf16, fp16 or SiLU-gated bf16.
+static int w4mm_reduce(const float *part, void *c, int M, int N, int splits, bool silu, bool f16, void *stream) {
+  using namespace cfa::abi;
+  using namespace cfa::w4mm;
+  hipStream_t st = (hipStream_t)stream;
+  const long long MN = (long long)M * N;
+  if (f16) return cfa::w4few::reduce_f16(part, c, MN, splits, stream);
+  if (silu) {
+    const long long MF = MN / 2;  // N % 64 == 0: four features per thread
+    CFA_LAUNCH("w4a16_gemm_zp_reduce", w4mm_reduce_silu_kernel, dim3((unsigned)((MF / 4 + 255) / 256)), dim3(256),
+               0, st, part, (uint16_t *)c, M, N, splits);
+  } else {
+    CFA_LAUNCH("w4a16_gemm_zp_reduce", w4mm_reduce_kernel, dim3((unsigned)((MN / 4 + 255) / 256)), dim3(256), 0,
+               st, part, (uint16_t *)c, MN, splits);
+  }
+  return CFA_OK;
+}
+
+// Few rows, any of the modes below.
+static int few_launch(const void *a, const uint32_t *b_quant, const void *scales, const void *zeros, int M, int N,
+                      int K, int group, int form, void *c, void *workspace, size_t workspace_bytes, void *stream,
+                      int mode) {
+  using namespace cfa::abi;
+  namespace few = cfa::w4few;
+  const int S = few::splits(M, N, K);
+  const bool part = S > 1 || mode == 2;
+  const size_t need = part ? (size_t)S * M * N * sizeof(float) : 0;
+  if (need && (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 15) != 0))
+    return fail_arg(mode == 2 ? "part too small (cfa_w4a16_gemm_zp_splits x M x N fp32)"
+                              : "workspace too small (see cfa_w4a16_gemm_zp_workspace_size)");
+  if (int rc = few::launch(a, b_quant, scales, zeros, M, N, K, group, form, c, (float *)workspace, S, part ? 2 : mode,
+                           stream))
+    return rc;
+  if (mode == 2 || S == 1) return CFA_OK;
+  return w4mm_reduce((const float *)workspace, c, M, N, S, mode == 1, form == 2, stream);
 }
 
 // mode: 0 bf16 C, 1 SiLU-gated bf16 C, 2 fp32 partials only (in workspace)
@@ -451,6 +497,9 @@ static int w4mm_launch(const void *a, const uint32_t *b_quant, const void *scale
   if (!a || !b_quant || !scales || (!c && !part_only)) return fail_arg("null pointer");
   if ((((uintptr_t)a | (uintptr_t)c | (uintptr_t)b_quant | (uintptr_t)scales | (uintptr_t)zeros) & 15) != 0)
     return fail_arg("a, b_quant, scales, zeros and c must be 16-byte aligned");
+  if (few_rows(M, N, K))
+    return few_launch(a, b_quant, scales, zeros, M, N, K, group_size, 1, c, workspace, workspace_bytes, stream,
+                      mode);
   int spp = 0;
   if ((long long)M * K >= (1LL << 31)) return fail_arg("M * K must be below 2^31");
   const int splits = choose_splits(M, N, K, device_cu_count(), &spp);
@@ -481,16 +530,7 @@ static int w4mm_launch(const void *a, const uint32_t *b_quant, const void *scale
   CFA_LAUNCH(silu ? "w4a16_gemm_zp_silu" : "w4a16_gemm_zp", w4mm_kernel,
              dim3((unsigned)blocks, 1, (unsigned)splits), dim3(kNT), 0, st, g);
   if (part_only) return CFA_OK;
-  if (splits > 1 && silu) {
-    const long long MF = (long long)M * (N / 2);  // N % 256 == 0: four features per thread
-    CFA_LAUNCH("w4a16_gemm_zp_reduce", w4mm_reduce_silu_kernel,
-               dim3((unsigned)((MF / 4 + 255) / 256)), dim3(256), 0, st, (const float *)workspace,
-               (uint16_t *)c, M, N, splits);
-  } else if (splits > 1) {
-    const long long MN = (long long)M * N;  // N % 128 == 0: four columns per thread
-    CFA_LAUNCH("w4a16_gemm_zp_reduce", w4mm_reduce_kernel, dim3((unsigned)((MN / 4 + 255) / 256)),
-               dim3(256), 0, st, (const float *)workspace, (uint16_t *)c, MN, splits);
-  }
+  if (splits > 1) return w4mm_reduce((const float *)workspace, c, M, N, splits, silu, false, stream);
   return CFA_OK;
 }
 
@@ -511,7 +551,30 @@ extern "C" int cfa_w4a16_gemm_zp_silu(const void *a, const uint32_t *b_quant, co
 
 extern "C" int cfa_w4a16_gemm_zp_splits(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0 || N % cfa::w4mm::kBN != 0 || K % cfa::w4mm::kSK != 0) return 0;
-  return cfa::w4mm::choose_splits(M, N, K, cfa::abi::device_cu_count(), nullptr);
+  return cfa::w4mm::splits_of(M, N, K);
+}
+
+extern "C" size_t cfa_w4a16_gemm_few_workspace_size(int M, int N, int K) {
+  if (M <= 0 || M > cfa::w4few::kMaxM || N <= 0 || K <= 0 || N % 128 != 0 || K % 128 != 0) return 0;
+  const int s = cfa::w4few::splits(M, N, K);
+  return s > 1 ? (size_t)s * M * N * sizeof(float) : 0;
+}
+
+extern "C" int cfa_w4a16_gemm_few(const void *a, const uint32_t *b_quant, const void *scales, const void *zeros,
+                                  int M, int N, int K, int group_size, int is_fp16, void *c, void *workspace,
+                                  size_t workspace_bytes, void *stream) {
+  using namespace cfa::abi;
+  clear_error();
+  if (M <= 0 || M > cfa::w4few::kMaxM) return fail_arg("M must be in 1..128");
+  if (N <= 0 || N % 128 != 0) return fail_arg("N must be a positive multiple of 128");
+  if (K <= 0 || K % 128 != 0) return fail_arg("K must be a positive multiple of 128");
+  if (group_size <= 0 || group_size % 32 != 0 || K % group_size != 0)
+    return fail_arg("group_size must be a multiple of 32 that divides K");
+  if (!a || !b_quant || !scales || !c) return fail_arg("null pointer");
+  if ((((uintptr_t)a | (uintptr_t)c | (uintptr_t)b_quant | (uintptr_t)scales | (uintptr_t)zeros) & 15) != 0)
+    return fail_arg("a, b_quant, scales, zeros and c must be 16-byte aligned");
+  return few_launch(a, b_quant, scales, zeros, M, N, K, group_size, is_fp16 ? 2 : 0, c, workspace, workspace_bytes,
+                    stream, 0);
 }
 
 extern "C" int cfa_w4a16_gemm_zp_partials(const void *a, const uint32_t *b_quant, const void *scales,

@@ -6,8 +6,9 @@
 (``csrc/include/cudaforge/kernels/dequantize.cuh:12-25``,
 ``tests/unit/test_int4_dequant.py:6-15``).  ``int4_gemm_dequant`` mirrors
 ``int4_gemm_dequant_triton`` (``csrc/kernels/triton/int4_dequant_triton.py:
-86-131``): ``cfa_w4a16_dequant_t`` (the dequantised matrix written as
-[N, K]) followed by a PyTorch-ROCm GEMM in the activations' dtype.  ``w4a16_gemm`` is the fused MFMA kernel
+86-131``): ``cfa_w4a16_gemm_few`` for at most 128 rows, else
+``cfa_w4a16_dequant_t`` (the dequantised matrix written as [N, K]) followed by
+a PyTorch-ROCm GEMM in the activations' dtype.  ``w4a16_gemm`` is the fused MFMA kernel
 (``cfa_w4a16_gemm``: dequantisation in registers, no zero points).
 """
 from __future__ import annotations
@@ -208,7 +209,8 @@ class W4A16Linear:
 
     # class-wide switches: `fused_zp` (default) multiplies with
     # cfa_w4a16_gemm_zp, which dequantises in LDS per output tile, where the
-    # shape allows (bf16, N % 256 == 0); at the verify step's M = 504 it takes
+    # shape allows (bf16, N % 256 == 0; at most 128 rows take a kernel of
+    # their own); at the verify step's M = 504 it takes
     # 51 / 42 / 150 / 85 us for QKV / O / gate-up / down against 51 / 43 / 175
     # / 110 us for dequantise + hipBLASLt.  `fused` selects the older
     # cfa_w4a16_gemm (no zero points) instead; off.
@@ -253,6 +255,28 @@ class W4A16Linear:
         return silu_mul(deinterleave_gate_up(self(x, scratch)).contiguous())
 
 
+def _few_rows_ok(a: torch.Tensor, b_quant: torch.Tensor, scales: torch.Tensor, zeros,
+                 group_size: int) -> bool:
+    """Whether int4_gemm_dequant's product runs on cfa_w4a16_gemm_few: at most
+    128 contiguous rows in shapes it takes (else dequantise + GEMM, which is
+    also the path that autograd and torch's function transforms see)."""
+    K, N = a.shape[1], b_quant.shape[1] if b_quant.dim() == 2 else 0
+    if type(a) is not torch.Tensor or (a.requires_grad and torch.is_grad_enabled()):
+        return False
+    if torch._C._functorch.peek_interpreter_stack() is not None \
+            or torch.autograd.forward_ad._current_level >= 0 \
+            or torch._C._len_torch_dispatch_stack() > 0:
+        return False
+    tensors = [a, b_quant, scales] + ([] if zeros is None else [zeros])
+    return (0 < a.shape[0] <= 128 and N > 0 and N % 128 == 0 and K % 128 == 0
+            and group_size > 0 and group_size % 32 == 0 and K % group_size == 0
+            and all(t.device == a.device and t.device.type == "cuda" and t.is_contiguous()
+                    and t.data_ptr() % 16 == 0 for t in tensors)
+            and b_quant.dtype == torch.int32
+            and all(t.dtype == torch.float16 and tuple(t.shape) == (K // group_size, N)
+                    for t in tensors[2:]))
+
+
 def int4_gemm_dequant(a: torch.Tensor, b_quant: torch.Tensor, scales: torch.Tensor,
                       zeros: Optional[torch.Tensor] = None, group_size: int = 128) -> torch.Tensor:
     """a [M, K] fp16 (or bf16) @ dequant(b_quant) -> [M, N] in a's dtype
@@ -261,6 +285,23 @@ def int4_gemm_dequant(a: torch.Tensor, b_quant: torch.Tensor, scales: torch.Tens
         raise ValueError("a must be [M, K] fp16 or bf16")
     if b_quant.shape[0] * 8 != a.shape[1]:
         raise ValueError("K of a and b_quant differ")
+    if _few_rows_ok(a, b_quant, scales, zeros, group_size):
+        # one kernel that reads the packed words once (M = 4, K = 4096, N =
+        # 14336, fp16: 17 us against 43 for writing the dequantised matrix and
+        # reading it back)
+        lib = _lib.load()
+        (M, K), N = a.shape, b_quant.shape[1]
+        out = torch.empty(M, N, dtype=a.dtype, device=a.device)
+        need = lib.cfa_w4a16_gemm_few_workspace_size(M, N, K)
+        ws = torch.empty(need, dtype=torch.uint8, device=a.device) if need else None
+        with torch.cuda.device(a.device):
+            rc = lib.cfa_w4a16_gemm_few(
+                a.data_ptr(), b_quant.data_ptr(), scales.data_ptr(),
+                zeros.data_ptr() if zeros is not None else None, M, N, K, group_size,
+                1 if a.dtype == torch.float16 else 0, out.data_ptr(),
+                ws.data_ptr() if need else None, need, _stream_ptr(a.device))
+        _lib.check(rc, "cfa_w4a16_gemm_few")
+        return out
     # dequantised as [N, K]: hipBLASLt multiplies a @ w^T about 20% faster
     # than a @ w at the verify step's shapes
     wt = w4a16_dequant(b_quant, scales, zeros, group_size=group_size, dtype=a.dtype,
