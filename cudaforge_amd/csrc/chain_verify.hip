@@ -123,7 +123,7 @@ struct Args {
   int NC;                 // chunks per row
   MwJob *jobs;            // [B]
   MwRes *res;             // [B]
-  float *csum_x, *csum_t; // [B, NC] approximate chunk sums
+  float *csum_x, *csum_t; // [B, NC] approximate chunk sums (csum_t per row group)
   MwChunk *crec;          // [2, B, NC]   chunk structure, per pass
   MwRec *trec;            // [2, B, NC*64] tile functions, per pass
   int *badcnt;            // [2, B]
@@ -131,6 +131,7 @@ struct Args {
   float *x0;              // [2, B, kMwChunk] chunk 0's element values per pass
   unsigned long long *flags;  // [B, NC] look-back words of the first exact pass
   unsigned long long *tsync;  // [B, 2] mw_tail_kernel: S published, CDF shares done
+  int lparts;             // log2 of the work-groups per job of mw_tail_kernel
   float *s0;              // [B] sum pass: the exact running value after chunk 0
   int mw_reset;           // the first statistics pass zeroes flags and badcnt
   float *rawtok;          // [R] head pass: a row's raw logit at its position's draft token
@@ -1651,7 +1652,9 @@ template <bool KEEP>
 __global__ __launch_bounds__(kMwNT) void mw_first_kernel(Args a, int decide) {
   __shared__ __align__(16) float xs0[kMwChunk];  // chunk 0's values and tile records
   __shared__ MwRec tr0[kMwChunkTiles];
-  const int b = blockIdx.y, lane = threadIdx.x & 63;
+  // (decide: one row group; its draws, plain ones if there are several, share
+  // the row's chunk sums)
+  const int b = decide ? blockIdx.y * a.draws : blockIdx.y, lane = threadIdx.x & 63;
   const int c0 = kMwCPW * (blockIdx.x * (kMwNT / 64) + (threadIdx.x >> 6));
   MwJob j;
   if (decide) {
@@ -1668,6 +1671,13 @@ __global__ __launch_bounds__(kMwNT) void mw_first_kernel(Args a, int decide) {
     }
     __syncthreads();
     j = sj;
+    if (blockIdx.x == 0)
+      for (int d = 1 + (int)threadIdx.x; d < a.draws; d += kMwNT) {
+        MwJob jd = sj;
+        jd.u = a.U[(long long)(b + d) * a.ustride];
+        a.jobs[b + d] = jd;
+        a.res[b + d] = MwRes{0.0f, 0, -1, 0};
+      }
   } else {
     j = py_job(a, b);
   }
@@ -1715,7 +1725,7 @@ __global__ __launch_bounds__(kMwNT) void mw_first_kernel(Args a, int decide) {
     st = wave_sum_f32(st);
     sx[h] = wave_sum_f32(sxh);
     if (lane == 0 && (h == 0 || two)) {
-      a.csum_t[(long long)b * a.NC + c0 + h] = st;
+      a.csum_t[(long long)(b / a.draws) * a.NC + c0 + h] = st;
       a.csum_x[(long long)b * a.NC + c0 + h] = sx[h];
     }
   }
@@ -1957,14 +1967,13 @@ __device__ __forceinline__ float mw_walk(const Args &a, int b, int pass, const M
   return s;
 }
 
-// Everything after the first exact pass, kMwTailWGs work-groups ("parts")
-// of kMwTailNT threads per job:
+// Everything after the first exact pass, 2^a.lparts work-groups ("parts") of
+// kMwTailNT threads per job (tail_lparts):
 //   1. part 0's wave 0 (the walker) walks the sum pass (residual draws)
 //      from chunk 1 on (the first pass walked chunk 0) and publishes S;
 //   2. the walker writes the CDF pass's records of chunk 0 and walks it;
 //      meanwhile the other waves of the job write the records of chunks
-//      1 .. NC - 1 (chunk c to wave (c - 1) % 63 + 1 of the job's 64), from
-//      entry values that one wave per part scans from the stored chunk sums;
+//      1 .. NC - 1 (in turn), from entry values that one wave per part scans from the stored chunk sums;
 //   3. the other parts report their shares done, and the walker walks the
 //      rest of the CDF pass.
 // A job's stages follow each other directly instead of in three launches
@@ -1985,8 +1994,6 @@ __device__ __forceinline__ float mw_walk(const Args &a, int b, int pass, const M
 // could still be filling a slot.
 constexpr int kMwTailNT = 1024;
 constexpr int kMwTailWaves = kMwTailNT / 64;
-constexpr int kMwTailWGs = 4;
-constexpr int kMwTailWorkers = kMwTailWGs * kMwTailWaves - 1;  // every wave but the walker
 constexpr long kMwTailSpins = 1l << 15;  // s_sleep(2) polls: about 2 ms
 constexpr unsigned long long kTsyncSet = 1ull << 63;  // a.tsync[2 b]: S is there
 
@@ -1995,11 +2002,10 @@ __device__ __forceinline__ unsigned long long ts_load(unsigned long long *p) {
 }
 
 // Job b and part of linear work-group index L: groups of 8 jobs take
-// 8 * kMwTailWGs consecutive indices, the parts of one job 8 apart.
-__device__ __forceinline__ void mw_tail_ids(int L, int &b, int &part) {
-  const int grp = L / (8 * kMwTailWGs), w = L % (8 * kMwTailWGs);
-  b = grp * 8 + (w % 8);
-  part = w / 8;
+// 8 * parts consecutive indices, the parts of one job 8 apart.
+__device__ __forceinline__ void mw_tail_ids(unsigned L, int lparts, int &b, int &part) {
+  b = (int)((L >> (3 + lparts)) * 8 + (L & 7));
+  part = (int)((L >> 3) & ((1u << lparts) - 1u));
 }
 
 template <bool KEEP>
@@ -2009,7 +2015,9 @@ __global__ __launch_bounds__(kMwTailNT) void mw_tail_kernel(Args a) {
   __shared__ float sS;
   __shared__ int sok;
   int b, part;
-  mw_tail_ids(blockIdx.x, b, part);
+  const int parts = 1 << a.lparts;
+  mw_tail_ids(blockIdx.x, a.lparts, b, part);
+  const int workers = parts * kMwTailWaves - 1;  // every wave but the walker
   if (b >= a.B) return;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const MwJob j = a.jobs[b];
@@ -2020,7 +2028,7 @@ __global__ __launch_bounds__(kMwTailNT) void mw_tail_kernel(Args a) {
   const bool resid = j.kind == kResid, summed = mw_summed<KEEP>(j);
   // a wave that does not walk scans the chunk sums of the CDF pass's row
   if (wave == 1) {
-    const float *csum = (summed ? a.csum_x : a.csum_t) + (long long)b * a.NC;
+    const float *csum = summed ? a.csum_x + (long long)b * a.NC : a.csum_t + (long long)(b / a.draws) * a.NC;
     float carry = 0.0f;
     for (int base = 0; base < a.NC; base += 64) {
       const float v = (base + lane < a.NC) ? csum[base + lane] : 0.0f;
@@ -2063,7 +2071,7 @@ __global__ __launch_bounds__(kMwTailNT) void mw_tail_kernel(Args a) {
   // approximate entry value of chunk c on the CDF pass's scale (a residual
   // job whose sum fell to the fallback draws from t: t's own chunk sums)
   auto entry = [&](int c) __attribute__((always_inline)) -> float {
-    if (resid && e.fn == 2) return mw_entry_prefix(a.csum_t + (long long)b * a.NC, c);
+    if (resid && e.fn == 2) return mw_entry_prefix(a.csum_t + (long long)(b / a.draws) * a.NC, c);
     return (e.fn == 1 || (KEEP && e.fn == 4)) ? Es[c] / e.S : Es[c];
   };
   // records of chunk c; a chunk surely past u gets a "skipped" record and no
@@ -2079,11 +2087,11 @@ __global__ __launch_bounds__(kMwTailNT) void mw_tail_kernel(Args a) {
     mw_tile_values(a, e, (long long)c * kMwChunkTiles + lane, x);
     mw_records_chunk(a, b, c, kPassCdf, j, E0, x, c == 0 ? L.tr : nullptr, c == 0 ? L.xs : nullptr);
   };
-  // worker gw = 16 part + wave (1 .. 16 kMwTailWGs - 1) writes chunks gw,
-  // gw + kMwTailWorkers, ...; the walker (gw = 0) writes chunk 0 and walks it
+  // worker gw = 16 part + wave (1 .. 16 parts - 1) writes chunks gw,
+  // gw + workers, ...; the walker (gw = 0) writes chunk 0 and walks it
   // at once, while the workers write the rest
   auto share_of = [&](int gw) __attribute__((always_inline)) {
-    for (int c = gw; c < a.NC; c += kMwTailWorkers) records(c);
+    for (int c = gw; c < a.NC; c += workers) records(c);
   };
   const int gw = part * kMwTailWaves + wave;
   float s0 = 0.0f;
@@ -2110,16 +2118,16 @@ __global__ __launch_bounds__(kMwTailNT) void mw_tail_kernel(Args a) {
     unsigned long long n = 0;
     for (long k = 0; k < kMwTailSpins; ++k) {
       n = ts_load(ts + 1);
-      if (n >= (unsigned long long)(kMwTailWGs - 1)) break;
+      if (n >= (unsigned long long)(parts - 1)) break;
       __builtin_amdgcn_s_sleep(2);
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    sok = (n >= (unsigned long long)(kMwTailWGs - 1)) ? 1 : 0;
+    sok = (n >= (unsigned long long)(parts - 1)) ? 1 : 0;
   }
   __syncthreads();
   const bool all_in = sok != 0;
   if (!all_in) {
-    for (int p = 1; p < kMwTailWGs; ++p) share_of(p * kMwTailWaves + wave);
+    for (int p = 1; p < parts; ++p) share_of(p * kMwTailWaves + wave);
     __syncthreads();
   }
   if (wave == 0) mw_walk(a, b, kPassCdf, j, e, L, all_in, true, s0, found0);
@@ -2347,6 +2355,21 @@ static int sel_slices(const Args &a, int groups) {
   const int room = a.NC * kMwChunkTiles * (int)sizeof(MwRec) / kSelBytes;
   return std::max(2, std::min({kSelMaxHG, room, (512 + groups - 1) / groups}));
 }
+// log2 of the work-groups per job of mw_tail_kernel: as many as leave one work-group per
+// CU (a CU's second one waits for the first, and the walker's CU does best
+// alone), at most 8, and at least 12 chunks each.  us per call, V = 128256:
+//   jobs            8 (cpp)  32 (cpp)  64 (cpp)  128 (plain)  256 (plain)
+//   1 part            90.6     120.8     147.6       65.9         81.8
+//   2                 74.4     103.1     129.4       56.3         86.1
+//   4                 67.9      94.7     123.9       65.0        103.0
+//   8                 62.8      94.1     138.1       76.7        125.0
+// and V = 32000 (32 chunks), 64 jobs, cpp: 65.6, 62.5, 65.8, 78.8.
+static int tail_lparts(int jobs, int NC) {
+  const int most = std::min({8, abi::device_cu_count() / jobs, NC / 12});
+  int l = 0;
+  while ((2 << l) <= most) ++l;
+  return l;
+}
 // Head positions of the two-pass statistics (cpp rules, logits): with the
 // ~0.7 per-position acceptance of typical draft models, 3 minimises the rows
 // the two passes read together.
@@ -2564,8 +2587,10 @@ static int run_pipeline(Args &a, bool vec, void *workspace, hipStream_t st, floa
   // (cpp rules: mw_first_kernel takes each sequence's decision itself)
   if (mode == CFA_MODE_GREEDY) CFA_LAUNCH("chain_decide", decide_kernel, dim3(B), dim3(64), 0, st, a);
   if (mode != CFA_MODE_GREEDY) {
-    const dim3 cg1((a.NC + kMwChunksPerWG - 1) / kMwChunksPerWG, B);   // two chunks per wave
-    const unsigned tail_wgs = (unsigned)(((B + 7) / 8) * 8 * kMwTailWGs);
+    const int jobs = mode == CFA_MODE_PYTHON ? B : B / a.draws;
+    const dim3 cg1((a.NC + kMwChunksPerWG - 1) / kMwChunksPerWG, jobs);   // two chunks per wave
+    a.lparts = tail_lparts(B, a.NC);
+    const unsigned tail_wgs = (unsigned)((B + 7) / 8 * 8) << a.lparts;
     if (mode == CFA_MODE_PYTHON) {
       if (K > 0 || a.HG == 0)
         CFA_LAUNCH("chain_decide", py_decide_kernel, dim3(R / a.rpb), dim3(64 * std::min(a.rpb, 16)), 0, st, a);

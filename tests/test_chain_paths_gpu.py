@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 import torch
 
+from cudaforge_amd.sampling import sample
 from cudaforge_amd.verify import chain_verify
 from oracle import oracle as O
 
@@ -68,3 +69,19 @@ def test_python_two_pass(device, V, case):
                     tok.cpu().numpy(), u.cpu().numpy(), 0.9)
     assert np.array_equal(a.tokens.cpu().numpy(), toks)
     assert {"accept": K, "last": K - 1}.get(case, int(a.accept_len[0])) == int(a.accept_len[0])
+
+
+@pytest.mark.parametrize("R,V,draws", [(1, 13000, 1), (2, 128256, 3), (20, 65537, 2), (70, 128256, 2),
+                                       (130, 30001, 2)])
+def test_draws_by_work_groups_per_job(device, R, V, draws):
+    """Multinomial draws with 1 to 8 work-groups per draw (by the number of
+    draws and the row's chunks); the draws of a row share its chunk sums."""
+    g = torch.Generator(device=device).manual_seed(R + V)
+    x = 2.0 * torch.randn(R, V, device=device, generator=g)
+    u = 1.0 - torch.rand(R, draws, device=device, generator=g)
+    u[0, 0], u[-1, -1] = 2.0 ** -24, 1.0
+    tok, p = sample(x, draws=draws, uniforms=u, return_probs=True)
+    for r in sorted({0, R // 2, R - 1}):
+        for d in range(draws):
+            assert tok[r, d].item() == O.sample_from_distribution(p[r].cpu().numpy(), float(u[r, d])), (r, d)
+    assert torch.equal(tok, sample(x, draws=draws, uniforms=u))
