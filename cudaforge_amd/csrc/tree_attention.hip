@@ -67,15 +67,20 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 constexpr int kKT = 64;                       // keys per tile
 constexpr int kWaves = 8;
 constexpr int kNT = kWaves * 64;              // threads per work-group
-constexpr int kQT = 2;                        // 16-row query tiles per wave
-constexpr int kMaxRows = kWaves * kQT * 16;   // 256 query rows per work-group
+// A wave owns QT 16-row query tiles: two, or one for at most 64 query rows
+// (then one wave per SIMD is busy either way, with half the work per tile: a
+// draft level of 8 sequences x 8 nodes, head_dim 64, 13.5 -> 12.3 us).  From
+// 65 to 128 rows one tile a wave would make all eight waves read every K and V
+// operand from LDS instead of four: 31 nodes at head_dim 128 39.4 -> 47.7 us.
+constexpr int kRowsOneTile = 64;
+constexpr int kMaxRows = kWaves * 2 * 16;     // query rows per work-group
 constexpr int kKStages = 4;                   // K-tile ring (tile u: stage u % 4)
 constexpr int kVStages = 5;                   // V-tile ring (read one iteration after K)
 constexpr float kRescaleSlack = 8.0f;         // log2 units
 
 // Layout constants of head size D (64 or 128): K / V rows of D bf16 values,
 // D / 8 16-byte chunks each.
-template <int D>
+template <int D, int QT = 2>
 struct Geo {
   static_assert(D == 64 || D == 128, "head_dim 64 or 128");
   static constexpr int kRowBytes = D * 2;             // one K or V row
@@ -85,7 +90,7 @@ struct Geo {
   static constexpr int kLoadsPerTile = 2 * (8 / kRowsPerLoad);  // K + V transfers per wave
   static constexpr int kKK = D / 32;                  // k-slices of the QK product
   static constexpr int kDT = D / 16;                  // 16-row blocks of O^T
-  static constexpr int kMfma = 2 * kDT * kQT + 2 * kQT + 4 * kKK * kQT;  // per MFMA phase
+  static constexpr int kMfma = 2 * kDT * QT + 2 * QT + 4 * kKK * QT;  // per MFMA phase
 };
 #ifndef CFA_TA_SGB
 #define CFA_TA_SGB 1
@@ -268,17 +273,19 @@ __device__ __forceinline__ float column_max(float v) {
 // Per-wave state of the pipelined loop: 16-row query tiles qt of this wave,
 // scores of one 64-key tile s[qt][blk][T] (keys blk*32 + 8g + 4T + i) and its
 // bf16 probabilities p[qt][blk] (keys blk*32 + 8g + 0..7).
+template <int QT>
 struct Scores {
-  f32x4 s[kQT][2][2];
+  f32x4 s[QT][2][2];
 };
+template <int QT>
 struct Probs {
-  bf16x8 p[kQT][2];
+  bf16x8 p[QT][2];
 };
 
-template <int D>
+template <int D, int QT>
 struct Lane {
-  bf16x8 qf[kQT][D / 32];  // Q^T columns pre-scaled by scale*log2(e)
-  uint64_t anc[kQT];       // ancestor-or-self masks of the wave's columns
+  bf16x8 qf[QT][D / 32];  // Q^T columns pre-scaled by scale*log2(e)
+  uint64_t anc[QT];       // ancestor-or-self masks of the wave's columns
   int koff[D / 32];        // K-tile LDS byte offsets of this lane's operand reads
   int vbase, vh;           // V-tile transposed-read offset and swizzle
   int g;                   // lane / 16
@@ -286,11 +293,11 @@ struct Lane {
 
 // S^T = K Q^T - base: the accumulators start at -b so that the products come
 // out relative to the column's exponent base.
-template <int D>
-__device__ __forceinline__ void qk_tile(const Lane<D> &ln, const uint8_t *Ks, const float *b,
-                                        Scores &S) {
+template <int D, int QT>
+__device__ __forceinline__ void qk_tile(const Lane<D, QT> &ln, const uint8_t *Ks, const float *b,
+                                        Scores<QT> &S) {
 #pragma unroll
-  for (int qt = 0; qt < kQT; ++qt)
+  for (int qt = 0; qt < QT; ++qt)
 #pragma unroll
     for (int blk = 0; blk < 2; ++blk)
 #pragma unroll
@@ -305,16 +312,17 @@ __device__ __forceinline__ void qk_tile(const Lane<D> &ln, const uint8_t *Ks, co
                                                           ln.koff[kk]);
         const bf16x8 kf = __builtin_bit_cast(bf16x8, kv);
 #pragma unroll
-        for (int qt = 0; qt < kQT; ++qt)
+        for (int qt = 0; qt < QT; ++qt)
           S.s[qt][blk][T] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, ln.qf[qt][kk], S.s[qt][blk][T], 0, 0, 0);
       }
 }
 
 // Online-softmax bookkeeping of one column: b is the exponent base (log2
 // units) the scores are relative to, valid says b has been set.
+template <int QT>
 struct Softmax {
-  float b[kQT];
-  bool valid[kQT];
+  float b[QT];
+  bool valid[QT];
 };
 
 // VALU phase of tile t: mask (tiles reaching the tree), column maxima, the
@@ -322,13 +330,13 @@ struct Softmax {
 // scores relative to each column's exponent base b; the base only moves when
 // a column's maximum exceeds it by more than kRescaleSlack, which also
 // rescales O and l (they hold tiles < t, so this precedes tile t's PV).
-template <int D>
-__device__ __forceinline__ void valu_phase(const Lane<D> &ln, int kbase, int ctx, Scores &S,
-                                           Softmax &sm, f32x4 (&o)[kQT][D / 16],
-                                           f32x4 (&lacc)[kQT], Probs &P) {
+template <int D, int QT>
+__device__ __forceinline__ void valu_phase(const Lane<D, QT> &ln, int kbase, int ctx, Scores<QT> &S,
+                                           Softmax<QT> &sm, f32x4 (&o)[QT][D / 16],
+                                           f32x4 (&lacc)[QT], Probs<QT> &P) {
   if (kbase + kKT > ctx) {
 #pragma unroll
-    for (int qt = 0; qt < kQT; ++qt) {
+    for (int qt = 0; qt < QT; ++qt) {
       // bit k: tile key k is visible to this column; this lane's keys are
       // blk*32 + 8g + 4T + i, i.e. bit blk*32 + 4T + i of vis >> 8g
       const uint64_t vis = tile_visibility(kbase, ctx, ln.anc[qt]) >> (8 * ln.g);
@@ -342,11 +350,11 @@ __device__ __forceinline__ void valu_phase(const Lane<D> &ln, int kbase, int ctx
                 ((vis >> (blk * 32 + 4 * T + i)) & 1ull) ? S.s[qt][blk][T][i] : -INFINITY;
     }
   }
-  float mx[kQT];
-  bool resc[kQT];
+  float mx[QT];
+  bool resc[QT];
   bool any = false;
 #pragma unroll
-  for (int qt = 0; qt < kQT; ++qt) {
+  for (int qt = 0; qt < QT; ++qt) {
     float v = -INFINITY;
 #pragma unroll
     for (int blk = 0; blk < 2; ++blk)
@@ -360,7 +368,7 @@ __device__ __forceinline__ void valu_phase(const Lane<D> &ln, int kbase, int ctx
   }
   if (__ballot(any) != 0) {
 #pragma unroll
-    for (int qt = 0; qt < kQT; ++qt) {
+    for (int qt = 0; qt < QT; ++qt) {
       const float d = resc[qt] ? mx[qt] : 0.0f;
       const float alpha = resc[qt] ? (sm.valid[qt] ? __builtin_amdgcn_exp2f(-d) : 0.0f) : 1.0f;
       sm.b[qt] += d;
@@ -375,7 +383,7 @@ __device__ __forceinline__ void valu_phase(const Lane<D> &ln, int kbase, int ctx
     }
   }
 #pragma unroll
-  for (int qt = 0; qt < kQT; ++qt)
+  for (int qt = 0; qt < QT; ++qt)
 #pragma unroll
     for (int blk = 0; blk < 2; ++blk)
 #pragma unroll
@@ -395,23 +403,23 @@ __device__ __forceinline__ void valu_phase(const Lane<D> &ln, int kbase, int ctx
 // issued right behind its predecessor stalls the matrix pipe.  Lane (g, col)
 // reads V rows blk*32 + 8g + 0..7 at d = dt*16 + col through two transposed
 // 4x16 reads.
-template <int D>
-__device__ __forceinline__ void mfma_phase(const Lane<D> &ln, const uint8_t *Knext, const uint8_t *Vs,
-                                           const float *b, const Probs &P, Scores &S,
-                                           f32x4 (&o)[kQT][D / 16], f32x4 (&lacc)[kQT]) {
+template <int D, int QT>
+__device__ __forceinline__ void mfma_phase(const Lane<D, QT> &ln, const uint8_t *Knext, const uint8_t *Vs,
+                                           const float *b, const Probs<QT> &P, Scores<QT> &S,
+                                           f32x4 (&o)[QT][D / 16], f32x4 (&lacc)[QT]) {
   constexpr int RB = Geo<D>::kRowBytes;
   bf16x8 ones;
 #pragma unroll
   for (int j = 0; j < 8; ++j) ones[j] = (__bf16)1.0f;
-  f32x4 negb[kQT];
+  f32x4 negb[QT];
 #pragma unroll
-  for (int qt = 0; qt < kQT; ++qt) negb[qt] = f32x4{-b[qt], -b[qt], -b[qt], -b[qt]};
+  for (int qt = 0; qt < QT; ++qt) negb[qt] = f32x4{-b[qt], -b[qt], -b[qt], -b[qt]};
   // the column sums first: they read no LDS, so they cover the latency of
   // the phase's first operand reads (about 1.5%)
 #pragma unroll
   for (int blk = 0; blk < 2; ++blk)
 #pragma unroll
-    for (int qt = 0; qt < kQT; ++qt)
+    for (int qt = 0; qt < QT; ++qt)
       lacc[qt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, P.p[qt][blk], lacc[qt], 0, 0, 0);
 #pragma unroll
   for (int blk = 0; blk < 2; ++blk) {
@@ -422,7 +430,7 @@ __device__ __forceinline__ void mfma_phase(const Lane<D> &ln, const uint8_t *Kne
       const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((CFA_LDS i16x4 *)(vp + 4 * RB));
       const bf16x8 vf = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
 #pragma unroll
-      for (int qt = 0; qt < kQT; ++qt)
+      for (int qt = 0; qt < QT; ++qt)
         o[qt][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, P.p[qt][blk], o[qt][dt], 0, 0, 0);
     }
   }
@@ -435,7 +443,7 @@ __device__ __forceinline__ void mfma_phase(const Lane<D> &ln, const uint8_t *Kne
         const bf16x8 kf = __builtin_bit_cast(
             bf16x8, *reinterpret_cast<const uint4 *>(Knext + (blk * 32 + T * 16) * RB + ln.koff[kk]));
 #pragma unroll
-        for (int qt = 0; qt < kQT; ++qt)
+        for (int qt = 0; qt < QT; ++qt)
           S.s[qt][blk][T] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
               kf, ln.qf[qt][kk], kk == 0 ? negb[qt] : S.s[qt][blk][T], 0, 0, 0);
       }
@@ -444,14 +452,14 @@ __device__ __forceinline__ void mfma_phase(const Lane<D> &ln, const uint8_t *Kne
   // reads after every pair of MFMAs
   __builtin_amdgcn_sched_group_barrier(0x0100, 8, 0);
 #pragma unroll
-  for (int j = 0; j < Geo<D>::kMfma / 2; ++j) {
+  for (int j = 0; j < Geo<D, QT>::kMfma / 2; ++j) {
     __builtin_amdgcn_sched_group_barrier(0x0008, 2, 0);
     __builtin_amdgcn_sched_group_barrier(0x0100, 2, 0);
   }
 #endif
 }
 
-template <int D>
+template <int D, int QT>
 __global__ __launch_bounds__(kNT) void tree_attn_kernel(Args a) {
   using Gm = Geo<D>;
   constexpr int kTileBytes = Gm::kTileBytes;
@@ -475,14 +483,14 @@ __global__ __launch_bounds__(kNT) void tree_attn_kernel(Args a) {
 
   // query rows of this wave: r = (node - q0) * G + head-in-group; Q^T is
   // scaled by scale*log2(e) once here so that scores come out in log2 units
-  Lane<D> ln;
+  Lane<D, QT> ln;
   ln.g = g;
-  bool qvalid[kQT];
+  bool qvalid[QT];
   {
     const uint64_t node_bits = a.N >= 64 ? ~0ull : ((1ull << a.N) - 1);
 #pragma unroll
-    for (int qt = 0; qt < kQT; ++qt) {
-      const int r = (wave * kQT + qt) * 16 + col;
+    for (int qt = 0; qt < QT; ++qt) {
+      const int r = (wave * QT + qt) * 16 + col;
       qvalid[qt] = r < a.rows;
       const int nl = qvalid[qt] ? r / a.G : 0, hg = r % a.G;
       ln.anc[qt] = qvalid[qt] ? a.mask[(long long)b * a.mask_sb + a.q0 + nl] & node_bits : 0ull;
@@ -526,11 +534,11 @@ __global__ __launch_bounds__(kNT) void tree_attn_kernel(Args a) {
   wait_vmcnt<0>();
   __syncthreads();
 
-  f32x4 o[kQT][D / 16];
-  f32x4 lacc[kQT];
-  Softmax sm;
+  f32x4 o[QT][D / 16];
+  f32x4 lacc[QT];
+  Softmax<QT> sm;
 #pragma unroll
-  for (int qt = 0; qt < kQT; ++qt) {
+  for (int qt = 0; qt < QT; ++qt) {
     sm.b[qt] = 0.0f;
     sm.valid[qt] = false;
     lacc[qt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -560,11 +568,11 @@ __global__ __launch_bounds__(kNT) void tree_attn_kernel(Args a) {
     // transfers' issue.
     const bool lag = wave >= kWaves / 2;
     if (lag) block_barrier();
-    Scores S;
-    Probs P;
+    Scores<QT> S;
+    Probs<QT> P;
     // a wave without query rows (few query nodes) only moves data and keeps
     // the barriers; its products would be discarded
-    const bool busy = wave * kQT * 16 < a.rows;  // wave-uniform
+    const bool busy = wave * QT * 16 < a.rows;  // wave-uniform
     if (busy) qk_tile(ln, kring, sm.b, S);
     for (int t = t0; t < t1; ++t) {
       const int kbase = t * kKT;
@@ -605,10 +613,10 @@ __global__ __launch_bounds__(kNT) void tree_attn_kernel(Args a) {
 
   // every lane holds its column's full sum; write final or partial outputs
 #pragma unroll
-  for (int qt = 0; qt < kQT; ++qt) {
+  for (int qt = 0; qt < QT; ++qt) {
     const float ls = lacc[qt][0];
     if (!qvalid[qt]) continue;
-    const int r = (wave * kQT + qt) * 16 + col;
+    const int r = (wave * QT + qt) * 16 + col;
     if (a.splits == 1) {
       const int nl = r / a.G, hg = r % a.G;
       uint16_t *op = a.out + (((long long)b * a.Nq + nl) * a.Hq + (long long)h * a.G + hg) * D;
@@ -736,6 +744,16 @@ static void split_plan(int B, int Hkv, int max_keys, int splits_req, int &splits
     const int cus = abi::device_cu_count();
     const int items = std::max(1, B * Hkv);
     s = std::max(1, (cus + items - 1) / items);  // about one work-group per compute unit
+    // ... each of at least five tiles (a split starts with the latency of its
+    // first transfers, and the ring holds three tiles ahead), but four splits
+    // of a short context are still faster than fewer.  us per call with the
+    // merge, 24 tiles, 24 (sequence, KV head) items: 8 splits 22.7, 4 20.4;
+    // 17 tiles of head_dim 64, 8 items: 17 splits 16.7, 4 11.9; 5 tiles, 8
+    // items: 1 split 12.5, 5 12.4, 3 11.1
+    s = std::min(s, std::max(4, tiles / 5));
+    // two splits of a handful of tiles cost more in the merge than they save
+    // (7 tiles, 128 items: 19.0 against 17.3)
+    if (s == 2 && tiles <= 8) s = 1;
   }
   // a split covers at most kMaxTilesPerSplit tiles (its page lookups fit LDS)
   s = std::max(s, (tiles + kMaxTilesPerSplit - 1) / kMaxTilesPerSplit);
@@ -822,13 +840,20 @@ extern "C" int cfa_tree_attention(const void *q, const void *k_pool, const void 
   hipStream_t st = (hipStream_t)stream;
   const dim3 grid(a.splits, n_kv_heads, B);
   const long long rows = (long long)B * n_kv_heads * a.rows;
+  const bool one = a.rows <= kRowsOneTile;
   if (head_dim == 128) {
-    CFA_LAUNCH("tree_attn", tree_attn_kernel<128>, grid, dim3(kNT), 0, st, a);
+    if (one)
+      CFA_LAUNCH("tree_attn", (tree_attn_kernel<128, 1>), grid, dim3(kNT), 0, st, a);
+    else
+      CFA_LAUNCH("tree_attn", (tree_attn_kernel<128, 2>), grid, dim3(kNT), 0, st, a);
     if (a.splits > 1)
       CFA_LAUNCH("tree_attn_merge", tree_merge_kernel<128>, dim3((unsigned)((rows + 15) / 16)),
                  dim3(256), 0, st, a);
   } else {
-    CFA_LAUNCH("tree_attn", tree_attn_kernel<64>, grid, dim3(kNT), 0, st, a);
+    if (one)
+      CFA_LAUNCH("tree_attn", (tree_attn_kernel<64, 1>), grid, dim3(kNT), 0, st, a);
+    else
+      CFA_LAUNCH("tree_attn", (tree_attn_kernel<64, 2>), grid, dim3(kNT), 0, st, a);
     if (a.splits > 1)
       CFA_LAUNCH("tree_attn_merge", tree_merge_kernel<64>, dim3((unsigned)((rows + 31) / 32)),
                  dim3(256), 0, st, a);
