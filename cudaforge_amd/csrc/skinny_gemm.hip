@@ -245,14 +245,26 @@ __global__ __launch_bounds__(256) void skinny_gemm_kernel(Args a) {
   __syncthreads();
   if (!last_flag) return;
   const float *all = a.part + (long long)tile * a.S * (4 * MT * 256);
-  for (int q = 0; q < a.S; ++q) {
+  // kQ splits' loads in flight at once: they miss every cache, and one split
+  // after another costs a memory latency each (the draft's 16 layers at 64
+  // rows, 2 to 8 splits: 1333 -> 1316 us a level)
+  constexpr int kQ = MT == 8 ? 2 : 4;
+  for (int q0 = 0; q0 < a.S; q0 += kQ) {
+    f32x4 v[kQ][MT];
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
+    for (int q = 0; q < kQ; ++q) {
+      const float *src = all + (long long)min(q0 + q, a.S - 1) * (4 * MT * 256) + wave * 256 + lane;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float v = __hip_atomic_load(all + (long long)q * (4 * MT * 256) + ((4 * i + wave) * 4 + e) * 64 + lane,
-                                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        sum[i][e] = q == 0 ? v : sum[i][e] + v;
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          v[q][i][e] = __hip_atomic_load(src + (16 * i + e) * 64, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+#pragma unroll
+    for (int q = 0; q < kQ; ++q)
+      if (q0 + q < a.S) {
+#pragma unroll
+        for (int i = 0; i < MT; ++i) sum[i] = q0 + q == 0 ? v[q][i] : sum[i] + v[q][i];
       }
   }
   finish(sum);
