@@ -497,11 +497,11 @@ static int w4mm_launch(const void *a, const uint32_t *b_quant, const void *scale
   if (!a || !b_quant || !scales || (!c && !part_only)) return fail_arg("null pointer");
   if ((((uintptr_t)a | (uintptr_t)c | (uintptr_t)b_quant | (uintptr_t)scales | (uintptr_t)zeros) & 15) != 0)
     return fail_arg("a, b_quant, scales, zeros and c must be 16-byte aligned");
+  if ((long long)M * K >= (1LL << 31)) return fail_arg("M * K must be below 2^31");
   if (few_rows(M, N, K))
     return few_launch(a, b_quant, scales, zeros, M, N, K, group_size, 1, c, workspace, workspace_bytes, stream,
                       mode);
   int spp = 0;
-  if ((long long)M * K >= (1LL << 31)) return fail_arg("M * K must be below 2^31");
   const int splits = choose_splits(M, N, K, device_cu_count(), &spp);
   const size_t need = (splits > 1 || part_only) ? (size_t)splits * M * N * sizeof(float) : 0;
   if (need && (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 15) != 0))
@@ -573,6 +573,7 @@ extern "C" int cfa_w4a16_gemm_few(const void *a, const uint32_t *b_quant, const 
   if (!a || !b_quant || !scales || !c) return fail_arg("null pointer");
   if ((((uintptr_t)a | (uintptr_t)c | (uintptr_t)b_quant | (uintptr_t)scales | (uintptr_t)zeros) & 15) != 0)
     return fail_arg("a, b_quant, scales, zeros and c must be 16-byte aligned");
+  if ((long long)M * K >= (1LL << 31)) return fail_arg("M * K must be below 2^31");
   return few_launch(a, b_quant, scales, zeros, M, N, K, group_size, is_fp16 ? 2 : 0, c, workspace, workspace_bytes,
                     stream, 0);
 }

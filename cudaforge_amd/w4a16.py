@@ -259,17 +259,19 @@ def _few_rows_ok(a: torch.Tensor, b_quant: torch.Tensor, scales: torch.Tensor, z
                  group_size: int) -> bool:
     """Whether int4_gemm_dequant's product runs on cfa_w4a16_gemm_few: at most
     128 contiguous rows in shapes it takes (else dequantise + GEMM, which is
-    also the path that autograd and torch's function transforms see)."""
+    also the path that autograd, autocast and torch's function transforms
+    see)."""
     K, N = a.shape[1], b_quant.shape[1] if b_quant.dim() == 2 else 0
     if type(a) is not torch.Tensor or (a.requires_grad and torch.is_grad_enabled()):
         return False
     if torch._C._functorch.peek_interpreter_stack() is not None \
             or torch.autograd.forward_ad._current_level >= 0 \
-            or torch._C._len_torch_dispatch_stack() > 0:
+            or torch._C._len_torch_dispatch_stack() > 0 \
+            or torch.is_autocast_enabled(a.device.type):
         return False
     tensors = [a, b_quant, scales] + ([] if zeros is None else [zeros])
-    return (0 < a.shape[0] <= 128 and N > 0 and N % 128 == 0 and K % 128 == 0
-            and group_size > 0 and group_size % 32 == 0 and K % group_size == 0
+    return (0 < a.shape[0] <= 128 and a.shape[0] * K < 2 ** 31 and K > 0 and N > 0 and N % 128 == 0
+            and K % 128 == 0 and group_size > 0 and group_size % 32 == 0 and K % group_size == 0
             and all(t.device == a.device and t.device.type == "cuda" and t.is_contiguous()
                     and t.data_ptr() % 16 == 0 for t in tensors)
             and b_quant.dtype == torch.int32

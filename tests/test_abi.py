@@ -197,3 +197,13 @@ def test_tree_status_check_raises_on_failures():
         check_status(torch.tensor([0, 0, 1, 0], dtype=torch.int32))
     with pytest.raises(RuntimeError, match=r"timed out .*\[0, 3\]"):
         check_status(torch.tensor([2, 0, 0, 2], dtype=torch.int32))
+
+
+@pytest.mark.parametrize("name", ["cfa_w4a16_gemm_zp", "cfa_w4a16_gemm_few"])
+def test_few_row_gemm_refuses_2_31_activations(name):
+    # the kernel's lane offsets into A are 32-bit byte offsets
+    lib = _lib.load()
+    mid = [0] if name.endswith("few") else []
+    rc = getattr(lib, name)(16, 16, 16, 16, 128, 256, 2 ** 24, 128, *mid, 16, None, 0, None)
+    assert rc == _lib.CFA_ERR_ARG
+    assert "below 2^31" in _lib.last_error()

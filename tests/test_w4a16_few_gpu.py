@@ -68,6 +68,8 @@ def test_other_calls_keep_their_path(device):
     assert torch.allclose(int4_gemm_dequant(wide[:, ::2], q, s, z), want, atol=2e-3, rtol=2e-3)
     v = torch.func.vmap(lambda r: int4_gemm_dequant(r, q, s, z))(a.view(2, 4, 256))
     assert torch.allclose(v.reshape(8, 256), want, atol=2e-3, rtol=2e-3)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert int4_gemm_dequant(a, q, s, z).dtype == torch.bfloat16
     with pytest.raises(ValueError):
         int4_gemm_dequant(a, q, s.float(), z)
     lib = _lib.load()
