@@ -45,6 +45,26 @@ def test_rmsnorm(device, with_delta):
     assert err <= 2 * ULP, err
 
 
+@pytest.mark.parametrize("d", [8, 1032, 2040, 2048, 2056, 4088, 4096, 4104])
+@pytest.mark.parametrize("with_delta", [False, True])
+def test_rmsnorm_row_lengths(device, d, with_delta):
+    """Edges of the register-held rows (2048 and 4096 elements) and the loop
+    for longer ones: the same tolerance as above."""
+    g = torch.Generator().manual_seed(d)
+    h = torch.randn(3, d, generator=g).bfloat16()
+    delta = torch.randn(3, d, generator=g).bfloat16() if with_delta else None
+    w = (1 + 0.1 * torch.randn(d, generator=g)).bfloat16()
+    hd = h.to(device)
+    out = torch.empty_like(hd)
+    rmsnorm_(hd, delta.to(device) if with_delta else None, w.to(device), 1e-5, out)
+    hh = (h + delta) if with_delta else h
+    assert torch.equal(hd.cpu(), hh)
+    xf = hh.double()
+    ref = xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + 1e-5) * w.double()
+    err = ((out.cpu().double() - ref).abs() / ref.abs().clamp_min(1e-3)).max().item()
+    assert err <= 2 * ULP, err
+
+
 def test_silu_mul(device):
     M, F = 19, 3000
     gu = (3 * torch.randn(M, 2 * F, generator=torch.Generator().manual_seed(2))).bfloat16()
