@@ -29,7 +29,9 @@ _KINDS = {"probs": _lib.CFA_INPUT_PROBS, "logits": _lib.CFA_INPUT_LOGITS}
 
 
 def _stream_ptr(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    # the raw handle, without a torch.cuda.Stream object for every call
+    index = torch.cuda.current_device() if device.index is None else device.index
+    return torch._C._cuda_getCurrentRawStream(index)
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
