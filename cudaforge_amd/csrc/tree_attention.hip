@@ -107,12 +107,12 @@ struct Args {
   const uint64_t *mask;    // [N] or [B, N]
   long long mask_sb;
   uint16_t *out;           // [B, Nq, Hq, D]
-  uint16_t *part_o;        // [S, B, Hkv, rows, D] partial outputs O / l, bf16
+  uint16_t *part_o;        // [S, B, Hkv, rows, D] partial outputs O / l, bf16 (part_f32: O, fp32)
   float2 *part_ml;         // [S, B, Hkv, rows] (exponent base in log2 units, sum)
   int B, N, Hq, Hkv, G, rows;
   int q0, Nq;              // query nodes q0 .. N - 1 (Nq = N - q0 of them)
   int max_blocks, num_blocks, num_layers, layer, bs;
-  int splits, tiles_per_split;
+  int splits, tiles_per_split, part_f32;
   float scale_log2;        // sm_scale * log2(e)
 };
 
@@ -632,8 +632,15 @@ __global__ __launch_bounds__(kNT) void tree_attn_kernel(Args a) {
         *reinterpret_cast<uint2 *>(op + dt * 16 + 4 * g) = w;
       }
     } else {
-      // normalised partial in bf16 (the merge weighs it by its sum l)
       const long long prow = (((long long)split * a.B + b) * a.Hkv + h) * a.rows + r;
+      if (g == 0) a.part_ml[prow] = make_float2(sm.valid[qt] ? sm.b[qt] : -INFINITY, ls);
+      if (a.part_f32) {  // the sums as they are
+        float *pp = reinterpret_cast<float *>(a.part_o) + prow * D;
+#pragma unroll
+        for (int dt = 0; dt < D / 16; ++dt) *reinterpret_cast<f32x4 *>(pp + dt * 16 + 4 * g) = o[qt][dt];
+        continue;
+      }
+      // normalised partial in bf16 (the merge weighs it by its sum l)
       uint16_t *pp = a.part_o + prow * D;
       const float inv = (ls > 0.0f) ? 1.0f / ls : 0.0f;
 #pragma unroll
@@ -645,18 +652,17 @@ __global__ __launch_bounds__(kNT) void tree_attn_kernel(Args a) {
               ((uint32_t)__builtin_bit_cast(uint16_t, (__bf16)(o[qt][dt][3] * inv)) << 16);
         *reinterpret_cast<uint2 *>(pp + dt * 16 + 4 * g) = w;
       }
-      if (g == 0) a.part_ml[prow] = make_float2(sm.valid[qt] ? sm.b[qt] : -INFINITY, ls);
     }
   }
 }
 
 // Log-sum-exp merge of the splits: out = sum_s w_s l_s o_s / sum_s w_s l_s
-// with w_s = 2^(m_s - max m) and o_s the normalised bf16 partial; D / 8
-// threads per query row, eight d-values (one 16-byte load per split) per
-// thread, 2048 / D rows per work-group.  Up to kMergeRegs splits are loaded in
-// one round before any arithmetic.
+// with w_s = 2^(m_s - max m) and o_s the normalised bf16 partial, or (F32)
+// l_s o_s the fp32 one; D / 8 threads per query row, eight d-values (one or
+// two 16-byte loads per split) per thread, 2048 / D rows per work-group.  Up
+// to kMergeRegs splits are loaded in one round before any arithmetic.
 constexpr int kMergeRegs = 4;  // splits merged from registers in one round of loads
-template <int D>
+template <int D, bool F32>
 __global__ __launch_bounds__(256) void tree_merge_kernel(Args a) {
   constexpr int kTPR = D / 8;  // threads per row
   const long long row_g = (long long)blockIdx.x * (256 / kTPR) + threadIdx.x / kTPR;
@@ -670,24 +676,41 @@ __global__ __launch_bounds__(256) void tree_merge_kernel(Args a) {
   const long long prow0 = ((long long)b * a.Hkv + h) * a.rows + r;
   float L = 0.0f;
   float acc[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-  auto add = [&](float w, const uint4 &v) {
-    const uint32_t *vs = reinterpret_cast<const uint32_t *>(&v);
+  struct Part {
+    uint4 v[F32 ? 2 : 1];
+  };
+  auto load = [&](long long prow) {
+    Part p;
+    const uint8_t *src = reinterpret_cast<const uint8_t *>(a.part_o) + (prow * D + 8 * q8) * (F32 ? 4 : 2);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      acc[2 * j] += w * __uint_as_float(vs[j] << 16);
-      acc[2 * j + 1] += w * __uint_as_float(vs[j] & 0xffff0000u);
+    for (int k = 0; k < (F32 ? 2 : 1); ++k) p.v[k] = reinterpret_cast<const uint4 *>(src)[k];
+    return p;
+  };
+  auto add = [&](float w, float l, const Part &p) {
+    const uint32_t *vs = reinterpret_cast<const uint32_t *>(p.v);
+    const float wl = w * l;
+    L += wl;
+    if constexpr (F32) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) acc[j] += w * __uint_as_float(vs[j]);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        acc[2 * j] += wl * __uint_as_float(vs[j] << 16);
+        acc[2 * j + 1] += wl * __uint_as_float(vs[j] & 0xffff0000u);
+      }
     }
   };
   if (a.splits <= kMergeRegs) {
     // every split's (base, sum) and partial in flight at once
     float2 ml[kMergeRegs];
-    uint4 v[kMergeRegs];
+    Part v[kMergeRegs];
 #pragma unroll
     for (int s = 0; s < kMergeRegs; ++s) {
       if (s < a.splits) {
         const long long prow = prow0 + s * split_stride;
         ml[s] = a.part_ml[prow];
-        v[s] = *reinterpret_cast<const uint4 *>(a.part_o + prow * D + 8 * q8);
+        v[s] = load(prow);
       }
     }
     float M = -INFINITY;
@@ -696,13 +719,8 @@ __global__ __launch_bounds__(256) void tree_merge_kernel(Args a) {
       if (s < a.splits) M = fmaxf(M, ml[s].x);
     const float base = (M == -INFINITY) ? 0.0f : M;
 #pragma unroll
-    for (int s = 0; s < kMergeRegs; ++s) {
-      if (s < a.splits) {
-        const float w = __builtin_amdgcn_exp2f(ml[s].x - base) * ml[s].y;
-        L += w;
-        add(w, v[s]);
-      }
-    }
+    for (int s = 0; s < kMergeRegs; ++s)
+      if (s < a.splits) add(__builtin_amdgcn_exp2f(ml[s].x - base), ml[s].y, v[s]);
   } else {
     float M = -INFINITY;
     for (int s = 0; s < a.splits; ++s) M = fmaxf(M, a.part_ml[prow0 + s * split_stride].x);
@@ -711,10 +729,7 @@ __global__ __launch_bounds__(256) void tree_merge_kernel(Args a) {
     for (int s = 0; s < a.splits; ++s) {
       const long long prow = prow0 + s * split_stride;
       const float2 ml = a.part_ml[prow];
-      const uint4 v = *reinterpret_cast<const uint4 *>(a.part_o + prow * D + 8 * q8);
-      const float w = __builtin_amdgcn_exp2f(ml.x - base) * ml.y;
-      L += w;
-      add(w, v);
+      add(__builtin_amdgcn_exp2f(ml.x - base), ml.y, load(prow));
     }
   }
   const float inv = (L > 0.0f) ? 1.0f / L : 0.0f;
@@ -737,42 +752,58 @@ using namespace cfa::tree;
 
 static size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
-static void split_plan(int B, int Hkv, int max_keys, int splits_req, int &splits, int &tps) {
-  const int tiles = std::max(1, (max_keys + kKT - 1) / kKT);
-  int s = splits_req;
-  if (s <= 0) {
-    const int cus = abi::device_cu_count();
-    const int items = std::max(1, B * Hkv);
-    s = std::max(1, (cus + items - 1) / items);  // about one work-group per compute unit
-    // ... each of at least five tiles (a split starts with the latency of its
-    // first transfers, and the ring holds three tiles ahead), but four splits
-    // of a short context are still faster than fewer.  us per call with the
-    // merge, 24 tiles, 24 (sequence, KV head) items: 8 splits 22.7, 4 20.4;
-    // 17 tiles of head_dim 64, 8 items: 17 splits 16.7, 4 11.9; 5 tiles, 8
-    // items: 1 split 12.5, 5 12.4, 3 11.1
-    s = std::min(s, std::max(4, tiles / 5));
-    // two splits of a handful of tiles cost more in the merge than they save
-    // (7 tiles, 128 items: 19.0 against 17.3)
-    if (s == 2 && tiles <= 8) s = 1;
+// The splits of the keys, and the tiles each covers.  f32: the partials are
+// kept in fp32.  Each bf16 partial is rounded by itself, and fewer of them
+// average less of that out (relative error against 64 bits, one sequence of 8
+// nodes, 17 tiles of head_dim 64: 17 splits 0.0032, 4 splits 0.0033, 4 in fp32
+// 0.0029), so the automatic plan takes fewer splits than one work-group per
+// CU only in fp32 (`fewer`).  A workspace that holds only the bf16 partials of
+// one work-group per CU gets that plan instead.
+struct Plan {
+  int splits, tps;
+  bool f32;
+  size_t bytes(size_t rows, int D) const {  // rows: query rows of all (sequence, KV head) items
+    const size_t prows = splits * rows;
+    return splits == 1 ? 256 : align256(prows * D * (f32 ? 4 : 2)) + align256(prows * sizeof(float2));
   }
-  // a split covers at most kMaxTilesPerSplit tiles (its page lookups fit LDS)
-  s = std::max(s, (tiles + kMaxTilesPerSplit - 1) / kMaxTilesPerSplit);
-  s = std::min(s, tiles);
-  tps = (tiles + s - 1) / s;
-  splits = (tiles + tps - 1) / tps;
+};
+static Plan split_plan(int B, int Hkv, int max_keys, int splits_req, bool fewer) {
+  const int tiles = std::max(1, (max_keys + kKT - 1) / kKT);
+  auto plan = [&](int s) {
+    // a split covers at most kMaxTilesPerSplit tiles (its page lookups fit LDS)
+    s = std::max(s, (tiles + kMaxTilesPerSplit - 1) / kMaxTilesPerSplit);
+    s = std::min(s, tiles);
+    const int tps = (tiles + s - 1) / s;
+    return Plan{(tiles + tps - 1) / tps, tps, false};
+  };
+  if (splits_req > 0) return plan(splits_req);
+  const int cus = abi::device_cu_count();
+  const int items = std::max(1, B * Hkv);
+  int s = std::max(1, (cus + items - 1) / items);  // about one work-group per compute unit
+  const Plan most = plan(s);
+  if (!fewer) return most;
+  // ... each of at least five tiles (a split starts with the latency of its
+  // first transfers, and the ring holds three tiles ahead), but four splits
+  // of a short context are still faster than fewer.  us per call with the
+  // merge, 8 nodes, head_dim 64, one work-group per CU -> as here: 17 tiles, 8
+  // (sequence, KV head) items 15.4 -> 9.8; 24 tiles, 24 items 12.6 -> 10.9; 55
+  // tiles, 8 items 22.3 -> 14.2 (bf16 partials: 9.8, 10.9, 15.8)
+  s = std::min(s, std::max(4, tiles / 5));
+  // two splits of a handful of tiles cost more in the merge than they save
+  // (7 tiles, 128 items: 19.0 against 17.3)
+  if (s == 2 && tiles <= 8) s = 1;
+  Plan p = plan(s);
+  p.f32 = p.splits < most.splits;
+  return p;
 }
 
 extern "C" size_t cfa_tree_attention_workspace_size(int B, int N, int n_q_heads, int n_kv_heads,
                                                     int head_dim, int max_keys, int num_splits) {
   if (B <= 0 || N <= 0 || n_kv_heads <= 0 || n_q_heads <= 0 || (head_dim != 64 && head_dim != 128))
     return 0;
-  int splits = 1, tps = 1;
-  split_plan(B, n_kv_heads, max_keys, num_splits, splits, tps);
-  if (splits == 1) return 256;
-  const int G = n_q_heads / n_kv_heads;
-  const size_t rows = (size_t)G * N;
-  const size_t prows = (size_t)splits * B * n_kv_heads * rows;
-  return align256(prows * head_dim * sizeof(uint16_t)) + align256(prows * sizeof(float2));
+  const size_t rows = (size_t)B * n_kv_heads * (n_q_heads / n_kv_heads) * N;
+  return std::max(split_plan(B, n_kv_heads, max_keys, num_splits, true).bytes(rows, head_dim),
+                  split_plan(B, n_kv_heads, max_keys, num_splits, false).bytes(rows, head_dim));
 }
 
 extern "C" int cfa_tree_attention(const void *q, const void *k_pool, const void *v_pool,
@@ -827,36 +858,45 @@ extern "C" int cfa_tree_attention(const void *q, const void *k_pool, const void 
   a.layer = layer;
   a.bs = block_size;
   a.scale_log2 = sm_scale * 1.4426950408889634f;
-  split_plan(B, n_kv_heads, max_keys, num_splits, a.splits, a.tiles_per_split);
-  const size_t need = cfa_tree_attention_workspace_size(B, Nq, n_q_heads, n_kv_heads, head_dim,
-                                                        max_keys, num_splits);
-  if (a.splits > 1) {
-    if (!workspace || workspace_bytes < need)
+  const long long rows = (long long)B * n_kv_heads * a.rows;
+  Plan p = split_plan(B, n_kv_heads, max_keys, num_splits, true);
+  if (p.splits > 1 && workspace_bytes < p.bytes(rows, head_dim))
+    p = split_plan(B, n_kv_heads, max_keys, num_splits, false);
+  a.splits = p.splits;
+  a.tiles_per_split = p.tps;
+  a.part_f32 = p.f32 ? 1 : 0;
+  if (p.splits > 1) {
+    if (!workspace || workspace_bytes < p.bytes(rows, head_dim))
       return fail_arg("workspace too small (see cfa_tree_attention_workspace_size)");
-    const size_t prows = (size_t)a.splits * B * n_kv_heads * a.rows;
     a.part_o = (uint16_t *)workspace;
-    a.part_ml = (float2 *)((char *)workspace + align256(prows * head_dim * sizeof(uint16_t)));
+    a.part_ml = (float2 *)((char *)workspace + align256(p.splits * rows * head_dim * (p.f32 ? 4 : 2)));
   }
   hipStream_t st = (hipStream_t)stream;
   const dim3 grid(a.splits, n_kv_heads, B);
-  const long long rows = (long long)B * n_kv_heads * a.rows;
   const bool one = a.rows <= kRowsOneTile;
   if (head_dim == 128) {
     if (one)
       CFA_LAUNCH("tree_attn", (tree_attn_kernel<128, 1>), grid, dim3(kNT), 0, st, a);
     else
       CFA_LAUNCH("tree_attn", (tree_attn_kernel<128, 2>), grid, dim3(kNT), 0, st, a);
-    if (a.splits > 1)
-      CFA_LAUNCH("tree_attn_merge", tree_merge_kernel<128>, dim3((unsigned)((rows + 15) / 16)),
-                 dim3(256), 0, st, a);
   } else {
     if (one)
       CFA_LAUNCH("tree_attn", (tree_attn_kernel<64, 1>), grid, dim3(kNT), 0, st, a);
     else
       CFA_LAUNCH("tree_attn", (tree_attn_kernel<64, 2>), grid, dim3(kNT), 0, st, a);
-    if (a.splits > 1)
-      CFA_LAUNCH("tree_attn_merge", tree_merge_kernel<64>, dim3((unsigned)((rows + 31) / 32)),
-                 dim3(256), 0, st, a);
   }
+  if (a.splits == 1) return CFA_OK;
+#define CFA_MERGE(D, F32)                                                                      \
+  CFA_LAUNCH("tree_attn_merge", (tree_merge_kernel<D, F32>),                                   \
+             dim3((unsigned)((rows + 2048 / D - 1) / (2048 / D))), dim3(256), 0, st, a)
+  if (head_dim == 128 && p.f32)
+    CFA_MERGE(128, true);
+  else if (head_dim == 128)
+    CFA_MERGE(128, false);
+  else if (p.f32)
+    CFA_MERGE(64, true);
+  else
+    CFA_MERGE(64, false);
+#undef CFA_MERGE
   return CFA_OK;
 }

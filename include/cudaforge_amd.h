@@ -192,7 +192,10 @@ int cfa_sample(const float *rows, int64_t row_stride, int input_kind, int R, int
  *   tree_mask  uint64 per node (bit j: node j is an ancestor of, or is, the
  *              node), [N] shared (stride 0) or [B, N] (stride N)
  *   max_keys   host-side bound on ctx_len + N over the batch (plans the splits)
- *   num_splits key-range splits (0: automatic); splits > 1 need workspace
+ *   num_splits key-range splits (0: automatic); splits > 1 need workspace.
+ *              Automatic splits that are fewer than one work-group per CU keep
+ *              their partials in fp32; a workspace with room only for the
+ *              bf16 partials of one work-group per CU gets those instead
  *   out        [B, N - first_node, n_q_heads, head_dim] bf16
  * Query (node i, head hq) attends to context positions [0, ctx_len) and to
  * tree positions ctx_len + j with bit j of tree_mask[i]; scores scale by

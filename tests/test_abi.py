@@ -207,3 +207,19 @@ def test_few_row_gemm_refuses_2_31_activations(name):
     rc = getattr(lib, name)(16, 16, 16, 16, 128, 256, 2 ** 24, 128, *mid, 16, None, 0, None)
     assert rc == _lib.CFA_ERR_ARG
     assert "below 2^31" in _lib.last_error()
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_tree_attention_workspace_holds_one_split_per_cu(D):
+    """Whatever splits the automatic plan takes, the workspace holds the bf16
+    partials of one work-group per CU (256 here), which it can fall back to."""
+    lib = _lib.load()
+    rows = 4 * 31
+    for items in (8, 16, 24, 40, 64, 128, 200, 256, 512):
+        for tiles in list(range(1, 70)) + [256, 257, 300, 2000]:
+            s = min(max(1, -(-256 // items), -(-tiles // 256)), tiles)
+            s = -(-tiles // -(-tiles // s))
+            p = s * items * rows
+            want = 256 if s == 1 else -(-p * D * 2 // 256) * 256 + -(-p * 8 // 256) * 256
+            got = lib.cfa_tree_attention_workspace_size(items // 8, 31, 32, 8, D, 64 * tiles, 0)
+            assert want <= got <= 2 * want, (items, tiles, got, want)
