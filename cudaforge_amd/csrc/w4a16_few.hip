@@ -371,7 +371,6 @@ __global__ __launch_bounds__(kNT, 2) void w4few_kernel(Args a) {
 // (in pairs, whose A operands share 128-byte lines).  A is so small that it
 // hits the cache, and no barrier ties the waves together: gate/up at M = 1
 // 18.7 us against 22.9 with the ring (59 MB of words), down 13.7 against 17.
-constexpr int kRowM = 16;
 constexpr int kRowBN = 64;
 constexpr int kRowDepth = 4;
 template <int FORM>

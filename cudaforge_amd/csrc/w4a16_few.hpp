@@ -9,7 +9,15 @@ namespace w4few {
 
 constexpr int kMaxM = 128;
 
-// Splits of K for a shape (N % 128 == 0, K % 128 == 0).
+// Shapes the kernels take: w4few_kernel (17 rows and more) moves the words of
+// 16 word rows by 32-bit byte offsets, 64 N bytes and a line.
+constexpr int kRowM = 16;
+constexpr int kMaxN = 1 << 26;
+inline bool takes(int M, int N, int K) {
+  return M > 0 && M <= kMaxM && N > 0 && N % 128 == 0 && K > 0 && K % 128 == 0 && (M <= kRowM || N <= kMaxN);
+}
+
+// Splits of K for a shape that it takes.
 int splits(int M, int N, int K);
 
 // form: how the weights are formed (0 bf16 as cfa_w4a16_dequant, 1 bf16 as

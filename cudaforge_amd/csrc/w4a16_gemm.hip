@@ -415,9 +415,6 @@ __global__ __launch_bounds__(256) void w4mm_reduce_silu_kernel(const float *part
   *reinterpret_cast<uint2 *>(C + i) = o;
 }
 
-// Shapes the few-row kernel (w4a16_few.hip) takes.
-inline bool few_rows(int M, int N, int K) { return M <= w4few::kMaxM && N % 128 == 0 && K % 128 == 0; }
-
 // Splits of K: enough work-groups for every CU, each split at least 8
 // slices; *spp slices per split, and no split empty.
 int choose_splits(int M, int N, int K, int cus, int *spp) {
@@ -432,7 +429,7 @@ int choose_splits(int M, int N, int K, int cus, int *spp) {
 
 // The splits an entry point uses: those of the few-row kernel or of this one.
 int splits_of(int M, int N, int K) {
-  return few_rows(M, N, K) ? w4few::splits(M, N, K) : choose_splits(M, N, K, abi::device_cu_count(), nullptr);
+  return w4few::takes(M, N, K) ? w4few::splits(M, N, K) : choose_splits(M, N, K, abi::device_cu_count(), nullptr);
 }
 
 }  // namespace w4mm
@@ -498,7 +495,7 @@ static int w4mm_launch(const void *a, const uint32_t *b_quant, const void *scale
   if ((((uintptr_t)a | (uintptr_t)c | (uintptr_t)b_quant | (uintptr_t)scales | (uintptr_t)zeros) & 15) != 0)
     return fail_arg("a, b_quant, scales, zeros and c must be 16-byte aligned");
   if ((long long)M * K >= (1LL << 31)) return fail_arg("M * K must be below 2^31");
-  if (few_rows(M, N, K))
+  if (cfa::w4few::takes(M, N, K))
     return few_launch(a, b_quant, scales, zeros, M, N, K, group_size, 1, c, workspace, workspace_bytes, stream,
                       mode);
   int spp = 0;
@@ -555,7 +552,7 @@ extern "C" int cfa_w4a16_gemm_zp_splits(int M, int N, int K) {
 }
 
 extern "C" size_t cfa_w4a16_gemm_few_workspace_size(int M, int N, int K) {
-  if (M <= 0 || M > cfa::w4few::kMaxM || N <= 0 || K <= 0 || N % 128 != 0 || K % 128 != 0) return 0;
+  if (!cfa::w4few::takes(M, N, K)) return 0;
   const int s = cfa::w4few::splits(M, N, K);
   return s > 1 ? (size_t)s * M * N * sizeof(float) : 0;
 }
@@ -568,6 +565,7 @@ extern "C" int cfa_w4a16_gemm_few(const void *a, const uint32_t *b_quant, const 
   if (M <= 0 || M > cfa::w4few::kMaxM) return fail_arg("M must be in 1..128");
   if (N <= 0 || N % 128 != 0) return fail_arg("N must be a positive multiple of 128");
   if (K <= 0 || K % 128 != 0) return fail_arg("K must be a positive multiple of 128");
+  if (!cfa::w4few::takes(M, N, K)) return fail_arg("N must be at most 2^26 for more than 16 rows");
   if (group_size <= 0 || group_size % 32 != 0 || K % group_size != 0)
     return fail_arg("group_size must be a multiple of 32 that divides K");
   if (!a || !b_quant || !scales || !c) return fail_arg("null pointer");

@@ -271,6 +271,7 @@ def _few_rows_ok(a: torch.Tensor, b_quant: torch.Tensor, scales: torch.Tensor, z
         return False
     tensors = [a, b_quant, scales] + ([] if zeros is None else [zeros])
     return (0 < a.shape[0] <= 128 and a.shape[0] * K < 2 ** 31 and K > 0 and N > 0 and N % 128 == 0
+            and (a.shape[0] <= 16 or N <= 2 ** 26)
             and K % 128 == 0 and group_size > 0 and group_size % 32 == 0 and K % group_size == 0
             and all(t.device == a.device and t.device.type == "cuda" and t.is_contiguous()
                     and t.data_ptr() % 16 == 0 for t in tensors)

@@ -331,8 +331,8 @@ int cfa_w4a16_gemm_zp(const void *a, const uint32_t *b_quant, const void *scales
                       const void *zeros, int M, int N, int K, int group_size, void *c,
                       void *workspace, size_t workspace_bytes, void *stream);
 /* cfa_w4a16_gemm_zp for few rows (1 <= M <= 128; decode) in bf16 or fp16:
- * N % 128 == 0, K % 128 == 0, group_size a multiple of 32 that divides K,
- * every pointer 16-byte aligned.  The weights are bit for bit those of
+ * N % 128 == 0 (at most 2^26 for M > 16), K % 128 == 0, group_size a multiple
+ * of 32 that divides K, every pointer 16-byte aligned.  The weights are bit for bit those of
  * cfa_w4a16_dequant in the same type.
  * `workspace` holds cfa_w4a16_gemm_few_workspace_size bytes (0: none). */
 size_t cfa_w4a16_gemm_few_workspace_size(int M, int N, int K);

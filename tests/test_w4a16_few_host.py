@@ -1,0 +1,42 @@
+"""CPU tier: the rules by which shapes reach the few-row W4A16 GEMM
+(csrc/w4a16_few.hpp, compiled with g++) and its entry point's refusals."""
+import ctypes
+import os
+import subprocess
+
+import pytest
+
+from cudaforge_amd import _lib
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+SRC = os.path.join(HERE, "native", "w4a16_few_host.cpp")
+LIB = os.path.join(HERE, "native", "libw4a16_few_host.so")
+HDR = os.path.join(os.path.dirname(HERE), "cudaforge_amd", "csrc", "w4a16_few.hpp")
+
+
+@pytest.fixture(scope="module")
+def few():
+    if not os.path.exists(LIB) or os.path.getmtime(LIB) < max(os.path.getmtime(f) for f in (SRC, HDR)):
+        subprocess.run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", SRC, "-o", LIB], check=True)
+    return ctypes.CDLL(LIB)
+
+
+@pytest.mark.parametrize("M", [1, 16, 17, 128, 129])
+def test_word_offsets_fit_32_bits(few, M):
+    """Lane offsets of w4few_kernel: 4 * (row N + 4 l) bytes, row <= 15, l <=
+    31, and the 16 bytes from there.  Every N that 17 rows and more are taken
+    for has to keep them below 2^32; up to 16 rows no such offset is formed."""
+    assert few.few_takes(M, 256, 128) == (M <= 128)
+    for N in (2 ** 26, 2 ** 26 + 128, 71582720, 71582848, 2 ** 28, 2 ** 31 - 128):
+        fits = 4 * (15 * N + 4 * 31) + 16 <= 2 ** 32
+        assert few.few_takes(M, N, 128) <= (M <= 16 or fits)
+    assert few.few_takes(M, 2 ** 26, 128) == (M <= 128)
+    assert few.few_takes(M, 2 ** 31 - 128, 128) == (M <= 16)
+
+
+@pytest.mark.parametrize("M", [17, 128])
+def test_entry_refuses_wider_weights(M):
+    lib = _lib.load()
+    rc = lib.cfa_w4a16_gemm_few(16, 16, 16, 16, M, 2 ** 26 + 128, 128, 128, 0, 16, None, 0, None)
+    assert rc == _lib.CFA_ERR_ARG and "2^26" in _lib.last_error()
+    assert lib.cfa_w4a16_gemm_few_workspace_size(M, 2 ** 26 + 128, 128) == 0
