@@ -71,7 +71,7 @@ struct Args {
   int tiles;          // column tiles
   int steps;          // pipeline steps per split
   int spg;            // k-slices of 32 per scale group
-  uint32_t spg_inv;   // 2^32 / (k-slices of 32 per scale group), rounded up (0: one slice)
+  SliceDiv group_of;  // division by spg
   int out;            // Out
 };
 enum Out : int { kPlain = 0, kSilu = 1, kPart = 2 };
@@ -259,7 +259,7 @@ __global__ __launch_bounds__(kNT, 2) void w4few_kernel(Args a) {
         if (more) base[j] += x < MT * 4 ? kStep * 2 : wstep;
       } else {
         const uint32_t sl = 4u * (uint32_t)(u0 + iu) + 2u * (x - MT * 4 - kWBytes / 1024) + (lane >> 5);
-        const long long grp = __umulhi(sl, a.spg_inv) + (a.spg_inv == 0u ? sl : 0u);
+        const long long grp = slice_group(sl, a.group_of);
         const __half *t = (lane & 16) && a.z ? a.z : a.s;
         dma16(t + grp * a.N + n0 + 8 * (lane & 15), (CFA_LDS void *)dst);
       }
@@ -507,10 +507,8 @@ int cfa::w4few::launch(const void *a, const uint32_t *b_quant, const void *scale
   g.S = S;
   g.tiles = N / kBN;
   g.steps = (K / kStep + S - 1) / S;
-  // slice / spg = mulhi(slice, ceil(2^32 / spg)) for slice * spg < 2^32
-  const uint32_t spg = (uint32_t)(group / kSK);
-  g.spg = (int)spg;
-  g.spg_inv = spg == 1 ? 0u : (uint32_t)(((1ull << 32) + spg - 1) / spg);
+  g.spg = group / kSK;
+  g.group_of = slice_div((uint32_t)g.spg);
   g.out = out;
   const dim3 grid((unsigned)((g.tiles + 7) / 8 * 8), (unsigned)S);
   hipStream_t st = (hipStream_t)stream;

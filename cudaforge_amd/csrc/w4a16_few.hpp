@@ -4,6 +4,8 @@
 
 #include <stdint.h>
 
+#include "common.hpp"
+
 namespace cfa {
 namespace w4few {
 
@@ -15,6 +17,25 @@ constexpr int kRowM = 16;
 constexpr int kMaxN = 1 << 26;
 inline bool takes(int M, int N, int K) {
   return M > 0 && M <= kMaxM && N > 0 && N % 128 == 0 && K > 0 && K % 128 == 0 && (M <= kRowM || N <= kMaxN);
+}
+
+// The group of k-slice sl without a division: sl / d = mulhi(2 sl, mul) >>
+// shift with mul = ceil(2^(31 + shift) / d) and shift = ceil(log2 d), exact
+// for every d >= 1 and sl < 2^26 (K < 2^31): mul d = 2^(31 + shift) + e with
+// e < d <= 2^shift, so the product is at most sl e < 2^(26 + shift) too
+// large, below the 2^(31 + shift) / d of a quotient's step (the same number
+// with shift 0 and 2^32 was exact only for sl d < 2^32).
+struct SliceDiv {
+  uint32_t mul;
+  int shift;
+};
+inline SliceDiv slice_div(uint32_t d) {
+  int s = 0;
+  while ((1ull << s) < d) ++s;
+  return SliceDiv{(uint32_t)(((1ull << (31 + s)) + d - 1) / d), s};
+}
+CFA_HD uint32_t slice_group(uint32_t sl, SliceDiv d) {
+  return (uint32_t)(((uint64_t)(2u * sl) * d.mul) >> 32) >> d.shift;
 }
 
 // Splits of K for a shape that it takes.

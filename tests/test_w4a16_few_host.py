@@ -40,3 +40,20 @@ def test_entry_refuses_wider_weights(M):
     rc = lib.cfa_w4a16_gemm_few(16, 16, 16, 16, M, 2 ** 26 + 128, 128, 128, 0, 16, None, 0, None)
     assert rc == _lib.CFA_ERR_ARG and "2^26" in _lib.last_error()
     assert lib.cfa_w4a16_gemm_few_workspace_size(M, 2 ** 26 + 128, 128) == 0
+
+
+@pytest.mark.parametrize("spg", [1, 2, 3, 4, 5, 7, 127, 4099, 65535, 65537, 65900, 131071, 2 ** 20 + 1,
+                                 2 ** 25 - 1, 2 ** 25 + 1, 2 ** 26 - 1, 2 ** 26])
+def test_scale_group_of_a_slice(few, spg):
+    """slice / spg at every slice next to a multiple of spg, for K up to the
+    entry points' bound of 2^31 (2^26 slices); one slice into another group
+    would read past the scales (spg = 65900 at K = 2108800 did)."""
+    few.few_group.restype = few.few_group_wrong.restype = ctypes.c_uint32
+    top = 2 ** 26
+    assert few.few_group_wrong(0, min(top, 1 << 18), spg) == min(top, 1 << 18)
+    assert few.few_group_wrong(top - (1 << 18), top, spg) == top
+    step = max(1, top // spg // 3000)
+    for q in list(range(0, top // spg, step)) + [top // spg]:
+        for sl in (q * spg - 1, q * spg, q * spg + spg - 1):
+            if 0 <= sl < top:
+                assert few.few_group(sl, spg) == sl // spg
