@@ -475,16 +475,20 @@ __global__ __launch_bounds__(256) void w4few_reduce_f16_kernel(const float *part
 // As many splits as fill the CUs (one work-group each), of at least 4 steps;
 // w4row_kernel: enough for 192 work-groups of at least 128 k per wave
 // (unsplit from N = 12288 on, where the reduction would cost more than the
-// idle CUs).
+// idle CUs).  At most 16 of them, as w4a16_gemm.hip takes for more rows, so
+// that a workspace for more rows serves these too; past 16 the partials cost
+// more than the CUs give (us at M = 1 / 64 / 128, without and with the bound:
+// N = 1024, K = 14336 12.5 / 20.0 / 25.0 -> 10.9 / 17.1 / 22.4; N = 256, K =
+// 65536 22.7 / 68.4 / 88.5 -> 15.5 / 36.0 / 48.5).
 int splits(int M, int N, int K) {
   if (M <= kRowM) {
     int S = 1;
-    while (N / kRowBN * S < 192 && K / (2 * S * kWaves) >= 128) S *= 2;
+    while (S < kMaxSplits && N / kRowBN * S < 192 && K / (2 * S * kWaves) >= 128) S *= 2;
     return S;
   }
   const int tiles = N / kBN, steps = K / kStep;
   const int cus = abi::device_cu_count();
-  const int S = std::max(1, std::min(cus / tiles, steps / 4));
+  const int S = std::max(1, std::min({cus / tiles, steps / 4, kMaxSplits}));
   const int per = (steps + S - 1) / S;
   return (steps + per - 1) / per;
 }

@@ -10,6 +10,7 @@ namespace cfa {
 namespace w4few {
 
 constexpr int kMaxM = 128;
+constexpr int kMaxSplits = 16;
 
 // Shapes the kernels take: w4few_kernel (17 rows and more) moves the words of
 // 16 word rows by 32-bit byte offsets, 64 N bytes and a line.

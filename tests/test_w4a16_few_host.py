@@ -57,3 +57,19 @@ def test_scale_group_of_a_slice(few, spg):
         for sl in (q * spg - 1, q * spg, q * spg + spg - 1):
             if 0 <= sl < top:
                 assert few.few_group(sl, spg) == sl // spg
+
+
+def test_workspace_for_more_rows_serves_fewer():
+    """A buffer sized for a call's largest M (up to one 256-row tile) is large
+    enough for every smaller one, whichever kernel each takes."""
+    lib = _lib.load()
+    rows = (1, 4, 15, 16, 17, 32, 33, 63, 64, 65, 100, 127, 128, 129, 160, 200, 256)
+    for N in (256, 512, 768, 1024, 1280, 2048, 3072, 4096, 6144, 12288, 14336, 28672):
+        for K in (128, 256, 1024, 1152, 4096, 8192, 8320, 14336, 16384, 20480, 32768, 65536, 131072):
+            size = [lib.cfa_w4a16_gemm_zp_workspace_size(M, N, K) for M in rows]
+            assert size == sorted(size), (N, K, size)
+            part = [lib.cfa_w4a16_gemm_zp_splits(M, N, K) * M for M in rows]
+            assert part == sorted(part), (N, K, part)
+            assert max(lib.cfa_w4a16_gemm_zp_splits(M, N, K) for M in rows) <= 16
+            for M in rows[:13]:
+                assert lib.cfa_w4a16_gemm_few_workspace_size(M, N, K) <= 16 * 4 * M * N
