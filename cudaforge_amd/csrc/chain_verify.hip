@@ -915,7 +915,10 @@ __device__ int sel_find(SelLds &L, const Args &a, double &F, uint32_t &C, int &r
   }
   __syncthreads();
   constexpr int NW = NT / 64;
-  double fx = F + (fi - f);
+  // (the sum before this thread from its neighbour, not as fi - f, which is
+  // NaN where a bin holds an infinity and would hide the crossing)
+  const double fp = __shfl_up(fi, 1, 64);
+  double fx = F + (lane ? fp : 0.0);
   uint32_t cx = C + (ci - c);
 #pragma unroll
   for (int w = 0; w < NW; ++w) {

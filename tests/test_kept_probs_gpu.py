@@ -61,3 +61,47 @@ def test_filtered_many_rows_repeat(device):
     assert torch.equal(a, b)
     for r in (0, 137, 299):
         assert a[r, 0].item() == O.sample_filtered(p[r].cpu().numpy(), float(u[r, 0]), 0.9, 0)
+
+
+@pytest.mark.parametrize("V", [1500, 50001])
+@pytest.mark.parametrize("top_p,top_k", [(0.9, 0), (0.9, 3), (1.0, 1), (1.0, 0)])
+def test_infinite_and_nan_probabilities(device, V, top_p, top_k):
+    """An infinite probability is the largest one; NaN is never kept (the
+    oracle, which sorts, gets a zero in its place)."""
+    g = torch.Generator().manual_seed(V)
+    x = torch.rand(6, V, generator=g) * 4.0 / V
+    x[0, V // 3] = float("inf")
+    x[1, V // 3] = x[1, V - 2] = float("inf")
+    x[2, 5] = float("nan")
+    x[3, ::7] = float("nan")
+    x[4] = float("nan")
+    x[5, 7], x[5, 9] = float("inf"), float("nan")
+    u = torch.rand(6, 3, generator=g)
+    u[:, 0], u[:, 1] = 0.0, LAST
+    tok = sample(x.to(device), mode="filtered", top_p=top_p, top_k=top_k, draws=3,
+                 uniforms=u.to(device), input_kind="probs").cpu().numpy()
+    for r in range(6):
+        p = torch.nan_to_num(x[r], nan=0.0, posinf=float("inf")).numpy()
+        for d in range(3):
+            assert tok[r, d] == O.sample_filtered(p, float(u[r, d]), top_p, top_k), (r, d)
+
+
+@pytest.mark.parametrize("V", [1500, 50001])
+def test_masked_and_broken_logits(device, V):
+    """-inf masks entries out; a row whose softmax is undefined (NaN, +inf,
+    or nothing but -inf) keeps nothing and falls to its last index."""
+    g = torch.Generator().manual_seed(V)
+    x = 2.0 * torch.randn(5, V, generator=g)
+    x[0, ::2] = float("-inf")
+    x[1] = float("-inf")
+    x[1, V // 2] = -3.0
+    x[2, 11] = float("nan")
+    x[3, 11] = float("inf")
+    x[4] = float("-inf")
+    u = torch.rand(5, 1, generator=g)
+    tok, p = sample(x.to(device), mode="filtered", top_p=0.9, top_k=50, uniforms=u.to(device),
+                    return_probs=True)
+    tok, p = tok.cpu().numpy(), p.cpu().numpy()
+    assert tok[0, 0] == O.sample_filtered(p[0], float(u[0, 0]), 0.9, 50) and tok[0, 0] % 2 == 1
+    assert tok[1, 0] == V // 2
+    assert (tok[2:, 0] == V - 1).all()
