@@ -54,8 +54,8 @@ def test_zp_entry_same_weights(device, M, N, K):
 
 
 def test_other_calls_keep_their_path(device):
-    """Rows that need a gradient, strided rows, odd column counts and more
-    than 128 rows go through dequantise + GEMM, and give the same product."""
+    """Rows that need a gradient, strided rows, mapped and autocast calls go
+    through dequantise + GEMM, and give the same product."""
     a, q, s, z = _problem(8, 256, 256, 128, torch.float16, True, device, 1)
     want = int4_gemm_dequant(a, q, s, z)
     x = a.clone().requires_grad_()
@@ -74,3 +74,13 @@ def test_other_calls_keep_their_path(device):
         int4_gemm_dequant(a, q, s.float(), z)
     lib = _lib.load()
     assert lib.cfa_w4a16_gemm_few_workspace_size(129, 256, 256) == 0
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K", [(128, 256, 256), (129, 256, 256), (5, 192, 256), (130, 192, 256), (5, 256, 192)])
+def test_both_sides_of_the_row_and_column_rules(device, dtype, M, N, K):
+    """128 and 129 rows, column counts and depths that are no multiple of 128
+    (the dequantised product): the same tolerance on every route, the library
+    product's sums included."""
+    a, q, s, z = _problem(M, N, K, 64, dtype, True, device, M + N)
+    _check(int4_gemm_dequant(a, q, s, z, group_size=64), a, q, s, z, 64)
