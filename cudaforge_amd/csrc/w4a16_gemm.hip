@@ -469,8 +469,9 @@ static int few_launch(const void *a, const uint32_t *b_quant, const void *scales
   const bool part = S > 1 || mode == 2;
   const size_t need = part ? (size_t)S * M * N * sizeof(float) : 0;
   if (need && (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 15) != 0))
-    return fail_arg(mode == 2 ? "part too small (cfa_w4a16_gemm_zp_splits x M x N fp32)"
-                              : "workspace too small (see cfa_w4a16_gemm_zp_workspace_size)");
+    return fail_arg(mode == 2   ? "part too small (cfa_w4a16_gemm_zp_splits x M x N fp32)"
+                    : form == 1 ? "workspace too small (see cfa_w4a16_gemm_zp_workspace_size)"
+                                : "workspace too small (see cfa_w4a16_gemm_few_workspace_size)");
   if (int rc = few::launch(a, b_quant, scales, zeros, M, N, K, group, form, c, (float *)workspace, S, part ? 2 : mode,
                            stream))
     return rc;

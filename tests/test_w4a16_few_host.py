@@ -73,3 +73,15 @@ def test_workspace_for_more_rows_serves_fewer():
             assert max(lib.cfa_w4a16_gemm_zp_splits(M, N, K) for M in rows) <= 16
             for M in rows[:13]:
                 assert lib.cfa_w4a16_gemm_few_workspace_size(M, N, K) <= 16 * 4 * M * N
+
+
+@pytest.mark.parametrize("M", [4, 100])
+def test_small_workspace_names_the_entrys_own_size_function(M):
+    lib = _lib.load()
+    N, K = 384, 4096                       # not a width that cfa_w4a16_gemm_zp takes
+    need = lib.cfa_w4a16_gemm_few_workspace_size(M, N, K)
+    assert need > 0 and lib.cfa_w4a16_gemm_zp_workspace_size(M, N, K) == 0
+    rc = lib.cfa_w4a16_gemm_few(16, 16, 16, 16, M, N, K, 128, 0, 16, 16, need - 16, None)
+    assert rc == _lib.CFA_ERR_ARG and "cfa_w4a16_gemm_few_workspace_size" in _lib.last_error()
+    rc = lib.cfa_w4a16_gemm_zp(16, 16, 16, 16, M, 256, K, 128, 16, 16, 16, None)
+    assert rc == _lib.CFA_ERR_ARG and "cfa_w4a16_gemm_zp_workspace_size" in _lib.last_error()
