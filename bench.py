@@ -584,8 +584,7 @@ def main() -> int:
     _lib.profile_enable(False)
 
     kern = {}
-    for name in ("chain_stats_head", "chain_stats_tail", "chain_decide", "chain_plan",
-                 "chain_mw_first", "chain_mw_tail", "chain_finish"):
+    for name in ("chain_stats_head", "chain_stats_tail", "chain_mw_first", "chain_mw_tail"):
         n, ms = _lib.profile_query(name)
         kern[name] = ms / args.steps  # per step
     _lib.profile_reset()

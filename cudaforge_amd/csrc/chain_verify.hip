@@ -84,7 +84,7 @@ struct MwBad {  // a tile the walk will probably replay serially, with its value
   float x[kMwTile];
 };
 // What select_kernel found of a row's smallest kept probability v: it lies in
-// histogram bin `bin` (or is known: state kSelKnown, its bits in `bin`),
+// histogram bin `bin` (or is known: kSelKnown in `rules`, its bits in C),
 // F and C are the sum and the count of the probabilities in higher bins, and
 // the rules still open (bit 0 top-p, bit 1 top-k) are in `rules`.
 struct SelRow {
@@ -812,6 +812,9 @@ struct XKeepNorm {
 
 constexpr int kSelBins = 1024;
 constexpr int kSelShift = 20;
+// (a bin with more keys than this is read from the row instead, by every
+// work-group that needs v: 32 rows of 128256, top-p 0.9, normal logits of
+// standard deviation 0.5 105 us, 0.3 244; one row of 10^6, deviation 2, 1032)
 constexpr int kSelMaxList = 8192;
 constexpr int kSelNT = 1024;
 constexpr int kSelBytes = kSelBins * 12;  // a slice's bins in the workspace
@@ -2366,7 +2369,13 @@ static int sel_slices(const Args &a, int groups) {
 //   2                 74.4     103.1     129.4       56.3         86.1
 //   4                 67.9      94.7     123.9       65.0        103.0
 //   8                 62.8      94.1     138.1       76.7        125.0
-// and V = 32000 (32 chunks), 64 jobs, cpp: 65.6, 62.5, 65.8, 78.8.
+// and V = 32000 (32 chunks), 64 jobs, cpp: 65.6, 62.5, 65.8, 78.8.  More jobs
+// under the cpp rules (K = 8, V = 128256, most draws residual; the python
+// rules' order is the same):
+//   jobs         72     96    128    160    192    256    384
+//   1 part    164.0  204.5  232.6  255.2  302.3  371.7  551.8
+//   2         145.2  186.2  215.1  260.3  305.4  381.6  563.1
+//   4         157.9  198.9  230.5  271.7  324.3  414.7  618.2
 static int tail_lparts(int jobs, int NC) {
   const int most = std::min({8, abi::device_cu_count() / jobs, NC / 12});
   int l = 0;
@@ -2382,8 +2391,13 @@ constexpr int kHeadPositions = 3;
 constexpr int kPyHeadPositions = 1;
 // Below this many bytes of rows one pass over all of them is faster: the
 // second launch waits for the first and then for each row's partials, of
-// which few rows have many (B = 8, K = 5, V = 128256, 45 MB, cpp rules:
-// 67.8 us in one pass, 85 in two; B = 64, 361 MB: 140 against 124).
+// which few rows have many.  us per call in one pass / in two, V = 128256:
+//   MiB                  45       64       96      127      160      224      300
+//   cpp, K = 8      62 / 78  68 / 80  74 / 84  79 / 90  83 / 83  99 / 93  113 / 105
+//   cpp, K = 4      60 / 80  66 / 79  77 / 92  82 / 88  90 / 97 108 / 112 124 / 131
+//   python, K = 8   66 / 70  73 / 71  79 / 72  85 / 76  94 / 78 109 / 85  122 / 90
+// (the more positions behind the head, the earlier two passes win; python
+// mode's lock step would from about 55 MiB on).
 constexpr long long kTwoPassBytes = 128ll << 20;
 
 // Workspace layout (each region 256-byte aligned).

@@ -317,7 +317,7 @@ __global__ __launch_bounds__(kNT, 2) void w4few_kernel(Args a) {
   };
   // Every step issues one stage's transfers (past the split's end too, to
   // slots no longer read), so that the waits always count the same.  At step
-  // t, after the barrier, stage t + 1 has landed (kP - 2 later ones are in
+  // t, after the barrier, stage t + 1 has landed (kS - 2 later ones are in
   // flight) and every wave has read stage t into registers, which frees its
   // slot for stage t + kS; the wave reads stage t + 1's operands and
   // multiplies stage t's.

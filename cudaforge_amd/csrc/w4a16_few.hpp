@@ -9,6 +9,9 @@
 namespace cfa {
 namespace w4few {
 
+// Eight 16-row tiles, the most whose sums a wave's registers hold.  Gate/up of
+// the 8B target, us: M = 64 31, 65 42 (eight tiles from there), 128 43, and
+// 129 68 on w4a16_gemm.hip's 256-row tiles.
 constexpr int kMaxM = 128;
 constexpr int kMaxSplits = 16;
 

@@ -325,7 +325,10 @@ int cfa_w4a16_gemm(const void *a, const uint32_t *b_quant, const void *scales, i
  * b_quant 4-byte, scales and zeros 2-byte.  Splits K over the work-groups
  * when the output tiles alone leave CUs idle: the fp32 partials go to
  * `workspace` (cfa_w4a16_gemm_zp_workspace_size bytes, 0 when no split is
- * used) and are summed in split order, so results are reproducible. */
+ * used) and are summed in split order, so results are reproducible.
+ * At most 128 rows take the kernels of cfa_w4a16_gemm_few where K % 128 ==
+ * 0: a row's result depends (in the order of its fp32 sums) on whether the
+ * call has 1..16, 17..128 or more rows. */
 size_t cfa_w4a16_gemm_zp_workspace_size(int M, int N, int K);
 int cfa_w4a16_gemm_zp(const void *a, const uint32_t *b_quant, const void *scales,
                       const void *zeros, int M, int N, int K, int group_size, void *c,
