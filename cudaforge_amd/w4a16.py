@@ -17,6 +17,8 @@ import math
 from typing import Optional
 
 import torch
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 from . import _lib
 from .verify import _stream_ptr
@@ -258,15 +260,18 @@ class W4A16Linear:
 def _few_rows_ok(a: torch.Tensor, b_quant: torch.Tensor, scales: torch.Tensor, zeros,
                  group_size: int) -> bool:
     """Whether int4_gemm_dequant's product runs on cfa_w4a16_gemm_few: at most
-    128 contiguous rows in shapes it takes (else dequantise + GEMM, which is
-    also the path that autograd, autocast and torch's function transforms
-    see)."""
+    128 contiguous rows in shapes it takes (else dequantise + GEMM, whose
+    product is also what autograd, autocast, a trace, torch's function
+    transforms and modes see)."""
     K, N = a.shape[1], b_quant.shape[1] if b_quant.dim() == 2 else 0
     if type(a) is not torch.Tensor or (a.requires_grad and torch.is_grad_enabled()):
         return False
     if torch._C._functorch.peek_interpreter_stack() is not None \
             or torch.autograd.forward_ad._current_level >= 0 \
             or torch._C._len_torch_dispatch_stack() > 0 \
+            or torch._C._get_tracing_state() is not None \
+            or (torch._C._len_torch_function_stack() > 0
+                and any(type(m) is not DeviceContext for m in _get_current_function_mode_stack())) \
             or torch.is_autocast_enabled(a.device.type):
         return False
     tensors = [a, b_quant, scales] + ([] if zeros is None else [zeros])

@@ -84,3 +84,29 @@ def test_both_sides_of_the_row_and_column_rules(device, dtype, M, N, K):
     product's sums included."""
     a, q, s, z = _problem(M, N, K, 64, dtype, True, device, M + N)
     _check(int4_gemm_dequant(a, q, s, z, group_size=64), a, q, s, z, 64)
+
+
+def test_traces_and_function_modes_see_the_product(device):
+    """A recorded trace holds the product of its input (an opaque kernel's
+    output would be left out), and a function mode is called for it; a device
+    context is no such mode."""
+    from torch.overrides import TorchFunctionMode
+
+    a, q, s, z = _problem(4, 256, 256, 128, torch.float16, True, device, 2)
+    want = int4_gemm_dequant(a, q, s, z)
+    traced = torch.jit.trace(lambda x: int4_gemm_dequant(x, q, s, z), (a,), check_trace=False)
+    assert "aten::matmul" in str(traced.graph) or "aten::mm" in str(traced.graph)
+
+    class Seen(TorchFunctionMode):
+        names = []
+
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            self.names.append(getattr(func, "__name__", str(func)))
+            return func(*args, **(kwargs or {}))
+
+    with Seen():
+        got = int4_gemm_dequant(a, q, s, z)
+    assert any("matmul" in n for n in Seen.names), Seen.names
+    assert torch.allclose(got, want, atol=2e-3, rtol=2e-3)
+    with torch.device(device):
+        assert torch.equal(int4_gemm_dequant(a, q, s, z), want)
