@@ -2376,8 +2376,20 @@ static int sel_slices(const Args &a, int groups) {
 //   1 part    164.0  204.5  232.6  255.2  302.3  371.7  551.8
 //   2         145.2  186.2  215.1  260.3  305.4  381.6  563.1
 //   4         157.9  198.9  230.5  271.7  324.3  414.7  618.2
-static int tail_lparts(int jobs, int NC) {
-  const int most = std::min({8, abi::device_cu_count() / jobs, NC / 12});
+// `plain` is the share of draws that are expected to be plain beside residual
+// ones (a bonus row under the cpp rules).  They take one pass instead of two
+// and leave their CUs early, so they count as seven eighths, for four parts
+// or two of at least 20 chunks each.  cpp, V = 128256, 2 / 4 parts:
+//   K             1            2            3            4            5            8
+//   65 jobs  91.2/84.5  102.2/95.5  114.6/109.5  133.5/127.3  138.6/136.4  145.6/141.6
+//   68       87.7/83.6  104.8/102.1 117.7/114.2  133.2/130.4  139.7/139.7  142.3/152.7
+//   72       93.8/94.6  108.6/106.2 119.9/115.0  138.1/139.2  140.2/148.1  145.9/158.2
+// and V = 64000 (15 chunks a part), 68 jobs, K = 2 71.6/73.8, K = 4 92.3/96.3;
+// 1 / 2 parts, V = 128256, 129 jobs: 134.9/117.7 (K = 1) to 205.5/189.2 (5).
+static int tail_lparts(int jobs, int NC, double plain) {
+  const int cus = abi::device_cu_count();
+  int most = std::min({8, cus / jobs, NC / 12});
+  if (plain > 0.0) most = std::max(most, std::min({4, (int)(cus / (jobs * (1.0 - 0.125 * plain))), NC / 20}));
   int l = 0;
   while ((2 << l) <= most) ++l;
   return l;
@@ -2606,7 +2618,8 @@ static int run_pipeline(Args &a, bool vec, void *workspace, hipStream_t st, floa
   if (mode != CFA_MODE_GREEDY) {
     const int jobs = mode == CFA_MODE_PYTHON ? B : B / a.draws;
     const dim3 cg1((a.NC + kMwChunksPerWG - 1) / kMwChunksPerWG, jobs);   // two chunks per wave
-    a.lparts = tail_lparts(B, a.NC);
+    // about 0.7 of the drafts are accepted (see kHeadPositions)
+    a.lparts = tail_lparts(B, a.NC, mode == CFA_MODE_CPP && K > 0 ? std::pow(0.7, K) : 0.0);
     const unsigned tail_wgs = (unsigned)((B + 7) / 8 * 8) << a.lparts;
     if (mode == CFA_MODE_PYTHON) {
       if (K > 0 || a.HG == 0)

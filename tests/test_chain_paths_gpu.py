@@ -85,3 +85,17 @@ def test_draws_by_work_groups_per_job(device, R, V, draws):
         for d in range(draws):
             assert tok[r, d].item() == O.sample_from_distribution(p[r].cpu().numpy(), float(u[r, d])), (r, d)
     assert torch.equal(tok, sample(x, draws=draws, uniforms=u))
+
+
+@pytest.mark.parametrize("B,K,V", [(65, 1, 90001), (68, 2, 82000), (71, 1, 128256), (130, 2, 41003)])
+def test_parts_past_one_work_group_per_cu(device, B, K, V):
+    """Four parts (two from 129 sequences) per draw where plain and residual
+    draws mix, on both sides of the rule."""
+    tl, dl, tok, u = _inputs(B, K, V, B + V, device)
+    u = u[:, : K + 1].contiguous()
+    o = chain_verify(tl, dl, tok, u, mode="cpp", return_probs=True)
+    n, toks = _want("cpp", o.target_probs.cpu().numpy(), o.draft_probs.cpu().numpy(),
+                    tok.cpu().numpy(), u.cpu().numpy(), 1.0)
+    assert np.array_equal(o.accept_len.cpu().numpy(), n)
+    assert np.array_equal(o.tokens.cpu().numpy(), toks)
+    assert torch.equal(chain_verify(tl, dl, tok, u, mode="cpp").tokens, o.tokens)
