@@ -595,7 +595,7 @@ def main() -> int:
     # the whole step on the workload's algorithmic bytes (every logit once)
     step_gbs = ALG_BYTES / (ms_per_step * 1e-3) / 1e9
     head_t = traffic_from_profile("cfa::chain::stats_kernel<256, 4> (head)")
-    tail_t = traffic_from_profile("cfa::chain::stats_tail_kernel<256>")
+    tail_t = traffic_from_profile("cfa::chain::stats_tail_kernel<256, 4>")
 
     line = {
         "metric": METRIC,
